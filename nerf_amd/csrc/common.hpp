@@ -88,7 +88,7 @@ __device__ __forceinline__ LevelCell level_cell(const float p[3], uint32_t N) {
     for (int a = 0; a < 3; ++a) {
         const float x   = fminf(fmaxf(p[a], 0.0f), 1.0f);
         const float pos = x * s;
-        uint32_t i      = (uint32_t)floorf(pos);
+        uint32_t i      = (uint32_t)pos;  // pos >= 0: truncation is the floor
         i               = i >= N ? N - 1u : i;
         c.i0[a]         = i;
         c.w[a]          = pos - (float)i;
@@ -114,21 +114,30 @@ __device__ __forceinline__ float corner_weight(const LevelCell& c, uint32_t corn
     return (wx * wy) * wz;
 }
 
-// Hash encoding of one level of one point: features (a0, a1) as fp32.
-// Corner order, weights and accumulation order are those of the oracle.
-template <typename TableT>
-__device__ __forceinline__ void encode_level(const GridParams& g, const TableT* __restrict__ table, const float p[3], uint32_t level, uint32_t N, bool dense, float& a0, float& a1) {
-    const LevelCell c  = level_cell(p, N);
-    const TableT* base = table + (uint64_t)level * g.table_size * 2u;
-    uint32_t idx[8];
-#pragma unroll
-    for (uint32_t k = 0; k < 8u; ++k) idx[k] = corner_index(c, k, N, dense, g.table_size - 1u);
-    float v0[8], v1[8];
+// Weighted sum of a cell's 8 corner entries (fp16 pairs, corner order).
+// kFma: each product is added in one rounding (v_fma_mix_f32, which reads the
+// fp16 operand directly) instead of a conversion, a product and a sum, 16
+// instructions for 48: the march-sample kernels.  The others keep the
+// two-rounding sums of the oracle, which the encode outputs are compared with
+// bit for bit.
+template <bool kFma>
+__device__ __forceinline__ void corner_sum(const LevelCell& c, const uint32_t v[8], float& a0, float& a1) {
+    a0 = 0.0f;
+    a1 = 0.0f;
 #pragma unroll
     for (uint32_t k = 0; k < 8u; ++k) {
-        v0[k] = (float)base[2u * idx[k]];
-        v1[k] = (float)base[2u * idx[k] + 1u];
+        const half2_t e = __builtin_bit_cast(half2_t, v[k]);
+        const float w   = corner_weight(c, k);
+        if constexpr (kFma) {
+            a0 = __builtin_fmaf((float)e[0], w, a0);
+            a1 = __builtin_fmaf((float)e[1], w, a1);
+        } else {
+            a0 = a0 + w * (float)e[0];
+            a1 = a1 + w * (float)e[1];
+        }
     }
+}
+__device__ __forceinline__ void corner_sum_f32(const LevelCell& c, const float v0[8], const float v1[8], float& a0, float& a1) {
     a0 = 0.0f;
     a1 = 0.0f;
 #pragma unroll
@@ -256,61 +265,50 @@ bool make_occ_view(const NerfExtOccupancy& o, OccView& v);
 //     merging the odd-x cases whose entries happen to be adjacent measured
 //     no faster).
 // Same entries, weights and summation order as encode_level.
-template <typename TableT>
-__device__ __forceinline__ void load_entry_pair(const TableT* p, float q[4]) {
-    if constexpr (sizeof(TableT) == 4) {
-        float4 w;
-        __builtin_memcpy(&w, p, 16);
-        q[0] = w.x;
-        q[1] = w.y;
-        q[2] = w.z;
-        q[3] = w.w;
-    } else {
-        half4_t w;
-        __builtin_memcpy(&w, p, 8);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) q[k] = (float)w[k];
-    }
-}
-
-template <typename TableT, bool kHashPairs = true>
+template <typename TableT, bool kHashPairs = true, bool kFma = false>
 __device__ __forceinline__ void encode_level_xpair(const GridParams& g, const TableT* __restrict__ table, const float p[3], uint32_t level, uint32_t N, bool dense, float& a0, float& a1) {
     const LevelCell c  = level_cell(p, N);
     const TableT* base = table + (uint64_t)level * g.table_size * 2u;
+    // Entry pairs as loaded: (first entry, second entry), fp32 pairs or packed fp16.
+    constexpr bool kF32 = sizeof(TableT) == 4;
     float v0[8], v1[8];
+    uint32_t v[8];
 #pragma unroll
     for (uint32_t e = 0; e < 4u; ++e) {  // (y, z) edge e: corners 2e (x) and 2e + 1 (x + 1)
         const uint32_t i0 = corner_index(c, 2u * e, N, dense, g.table_size - 1u);
         const uint32_t i1 = corner_index(c, 2u * e + 1u, N, dense, g.table_size - 1u);
-        float q[4];
-        if (dense) {
-            load_entry_pair(base + 2u * i0, q);
-            v0[2u * e]      = q[0];
-            v1[2u * e]      = q[1];
-            v0[2u * e + 1u] = q[2];
-            v1[2u * e + 1u] = q[3];
-        } else if (kHashPairs && i1 == (i0 ^ 1u)) {
-            load_entry_pair(base + 2u * (i0 & ~1u), q);
-            const bool odd  = (i0 & 1u) != 0u;
-            v0[2u * e]      = odd ? q[2] : q[0];
-            v1[2u * e]      = odd ? q[3] : q[1];
-            v0[2u * e + 1u] = odd ? q[0] : q[2];
-            v1[2u * e + 1u] = odd ? q[1] : q[3];
+        const bool pair   = dense || (kHashPairs && i1 == (i0 ^ 1u));
+        const bool odd    = !dense && pair && (i0 & 1u) != 0u;
+        const uint32_t at = dense ? i0 : (i0 & ~1u);
+        if constexpr (kF32) {
+            float2 lo, hi;
+            if (pair) {
+                float4 w;
+                __builtin_memcpy(&w, base + 2u * at, 16);
+                lo = odd ? make_float2(w.z, w.w) : make_float2(w.x, w.y);
+                hi = odd ? make_float2(w.x, w.y) : make_float2(w.z, w.w);
+            } else {
+                __builtin_memcpy(&lo, base + 2u * i0, 8);
+                __builtin_memcpy(&hi, base + 2u * i1, 8);
+            }
+            v0[2u * e]      = lo.x;
+            v1[2u * e]      = lo.y;
+            v0[2u * e + 1u] = hi.x;
+            v1[2u * e + 1u] = hi.y;
         } else {
-            v0[2u * e]      = (float)base[2u * i0];
-            v1[2u * e]      = (float)base[2u * i0 + 1u];
-            v0[2u * e + 1u] = (float)base[2u * i1];
-            v1[2u * e + 1u] = (float)base[2u * i1 + 1u];
+            uint2 w;
+            if (pair) {
+                __builtin_memcpy(&w, base + 2u * at, 8);
+            } else {
+                __builtin_memcpy(&w.x, base + 2u * i0, 4);
+                __builtin_memcpy(&w.y, base + 2u * i1, 4);
+            }
+            v[2u * e]      = odd ? w.y : w.x;
+            v[2u * e + 1u] = odd ? w.x : w.y;
         }
     }
-    a0 = 0.0f;
-    a1 = 0.0f;
-#pragma unroll
-    for (uint32_t k = 0; k < 8u; ++k) {
-        const float w = corner_weight(c, k);
-        a0            = a0 + w * v0[k];
-        a1            = a1 + w * v1[k];
-    }
+    if constexpr (kF32) corner_sum_f32(c, v0, v1, a0, a1);
+    else corner_sum<kFma>(c, v, a0, a1);
 }
 
 // One level of one point per lane, with the x-neighbour corners of each
@@ -327,65 +325,83 @@ __device__ __forceinline__ void encode_level_xpair(const GridParams& g, const Ta
 // entries, weights and summation order as encode_level.
 __device__ __forceinline__ uint32_t pair_swap(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, false); }  // quad_perm [1, 0, 3, 2]
 
-template <typename TableT>
+// kWide: every load is 8 bytes (an fp32 entry, or the aligned pair that holds
+// an fp16 entry).  The L1 serves lanes that share a 64-byte segment together
+// only for loads of 8 bytes and more: an instruction whose lane pairs have a
+// segment each takes 37 cycles with 4-byte loads and 19 with 8-byte ones;
+// lanes that read a few contiguous runs between them take 5-16 cycles with
+// 4-byte loads and 16 with 8-byte ones (measured, L1-resident).
+typedef uint32_t entry_pair __attribute__((ext_vector_type(2), aligned(4)));
+
+template <typename TableT, bool kFma = false, bool kWide = true>
 __device__ __forceinline__ void encode_level_lanepair(const GridParams& g, const TableT* __restrict__ table, const float p[3], uint32_t level, uint32_t N, bool dense, float& a0, float& a1) {
     constexpr uint32_t kWords = sizeof(TableT) == 4 ? 2u : 1u;  // dwords per entry
     const LevelCell c = level_cell(p, N);
     const bool odd    = (threadIdx.x & 1u) != 0u;
     const uint32_t h  = odd ? 1u : 0u;
-    LevelCell ce, co;  // cells of the even and the odd lane's point
+    // The point's index terms per axis (x, then y and z times their primes or
+    // strides), computed once by its own lane and handed to both lanes of the
+    // pair (quad_perm [0, 0, 2, 2]: the even lane's point; [1, 1, 3, 3]: the
+    // odd lane's); the corner one further along an axis adds that axis' step.
+    const uint32_t stride = N + 1u;
+    const uint32_t sy = dense ? stride : nerf_math::kPrime2, sz = dense ? stride * stride : nerf_math::kPrime3;
+    const uint32_t own[3] = {c.i0[0], c.i0[1] * sy, c.i0[2] * sz};
+    uint32_t pe[3], po[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const uint32_t other = pair_swap(c.i0[a]);
-        ce.i0[a]             = odd ? other : c.i0[a];
-        co.i0[a]             = odd ? c.i0[a] : other;
+        pe[a] = (uint32_t)__builtin_amdgcn_mov_dpp((int)own[a], 0xA0, 0xf, 0xf, false);
+        po[a] = (uint32_t)__builtin_amdgcn_mov_dpp((int)own[a], 0xF5, 0xf, 0xf, false);
     }
-    const uint32_t mask    = g.table_size - 1u;
-    const uint32_t* base   = reinterpret_cast<const uint32_t*>(table + (uint64_t)level * g.table_size * 2u);
+    const uint32_t mask  = g.table_size - 1u;
+    const uint32_t* base = reinterpret_cast<const uint32_t*>(table + (uint64_t)level * g.table_size * 2u);
+    auto index = [&](const uint32_t q[3], uint32_t e) {  // corner 2e + h (x's prime is 1)
+        const uint32_t x = q[0] + h, y = q[1] + ((e & 1u) ? sy : 0u), z = q[2] + ((e & 2u) ? sz : 0u);
+        return dense ? x + y + z : (x ^ y ^ z) & mask;
+    };
     uint32_t ve[4][kWords], vo[4][kWords];
+    auto fetch = [&](uint32_t i, uint32_t* d) {
+        if constexpr (kWords == 1u && !kWide) {
+            d[0] = base[i];
+            return;
+        }
+        const entry_pair w = *reinterpret_cast<const entry_pair*>(base + (kWords == 2u ? 2u * i : i & ~1u));
+        if constexpr (kWords == 2u) {
+            d[0]           = w[0];
+            d[kWords - 1u] = w[1];
+        } else {
+            // A bit select: the compiler turns a conditional of the two words
+            // into an indexed read of a copy in scratch memory.
+            const uint32_t m = 0u - (i & 1u);
+            d[0]             = (w[1] & m) | (w[0] & ~m);
+        }
+    };
 #pragma unroll
-    for (uint32_t e = 0; e < 4u; ++e) {
-        const uint32_t ie = corner_index(ce, 2u * e + h, N, dense, mask);
+    for (uint32_t e = 0; e < 4u; ++e) fetch(index(pe, e), ve[e]);
 #pragma unroll
-        for (uint32_t w = 0; w < kWords; ++w) ve[e][w] = base[kWords * ie + w];
-    }
-#pragma unroll
-    for (uint32_t e = 0; e < 4u; ++e) {
-        const uint32_t io = corner_index(co, 2u * e + h, N, dense, mask);
-#pragma unroll
-        for (uint32_t w = 0; w < kWords; ++w) vo[e][w] = base[kWords * io + w];
-    }
+    for (uint32_t e = 0; e < 4u; ++e) fetch(index(po, e), vo[e]);
     float v0[8], v1[8];
+    uint32_t v[8];
 #pragma unroll
     for (uint32_t e = 0; e < 4u; ++e) {
         uint32_t lo[kWords], hi[kWords];  // corners 2e and 2e + 1 of this lane's point
 #pragma unroll
         for (uint32_t w = 0; w < kWords; ++w) {
             const uint32_t recv = pair_swap(odd ? ve[e][w] : vo[e][w]);
-            const uint32_t own  = odd ? vo[e][w] : ve[e][w];
-            lo[w]               = odd ? recv : own;
-            hi[w]               = odd ? own : recv;
+            lo[w]               = odd ? recv : ve[e][w];
+            hi[w]               = odd ? vo[e][w] : recv;
         }
-        if constexpr (sizeof(TableT) == 4) {
+        if constexpr (kWords == 2u) {
             v0[2u * e]      = __uint_as_float(lo[0]);
             v1[2u * e]      = __uint_as_float(lo[kWords - 1u]);
             v0[2u * e + 1u] = __uint_as_float(hi[0]);
             v1[2u * e + 1u] = __uint_as_float(hi[kWords - 1u]);
         } else {
-            v0[2u * e]      = (float)__builtin_bit_cast(half_t, (uint16_t)(lo[0] & 0xffffu));
-            v1[2u * e]      = (float)__builtin_bit_cast(half_t, (uint16_t)(lo[0] >> 16));
-            v0[2u * e + 1u] = (float)__builtin_bit_cast(half_t, (uint16_t)(hi[0] & 0xffffu));
-            v1[2u * e + 1u] = (float)__builtin_bit_cast(half_t, (uint16_t)(hi[0] >> 16));
+            v[2u * e]      = lo[0];
+            v[2u * e + 1u] = hi[0];
         }
     }
-    a0 = 0.0f;
-    a1 = 0.0f;
-#pragma unroll
-    for (uint32_t k = 0; k < 8u; ++k) {
-        const float w = corner_weight(c, k);
-        a0            = a0 + w * v0[k];
-        a1            = a1 + w * v1[k];
-    }
+    if constexpr (kWords == 2u) corner_sum_f32(c, v0, v1, a0, a1);
+    else corner_sum<kFma>(c, v, a0, a1);
 }
 
 // --------------------------------------------------------------- cameras
@@ -484,6 +500,9 @@ struct FieldInputs {
     // level-split encode writes (each XCD whole lines of its levels) instead
     // of features_out, and the MLP pass reads.
     uint32_t* features_lm;
+    // Hashed levels below this one are gathered by 4-byte loads (level-major
+    // kernel; fp16 table).
+    uint32_t narrow_end;
 };
 
 // Owning ray of evaluated sample j (stream index qs), per FieldInputs.

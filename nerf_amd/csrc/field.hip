@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, c
             }
         }
         float feat[8];
-        encode_quad(g, table, p, grp, feat);
+        encode_quad<TableT, kFromSamples>(g, table, p, grp, feat);
         const half8_t x = to_half8(feat);
         if (in.features_out && s < n) *reinterpret_cast<half8_t*>(in.features_out + (uint64_t)s * 32u + 8u * grp) = x;
         floatx4 o, c;
@@ -209,13 +209,18 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, c
 // pair.  On hashed levels the two lanes of a pair fetch the x-neighbour
 // corners of one sample in the same load instruction (encode_level_lanepair:
 // one 128-byte line per sample where a lane per sample asks for two), which
-// halves the cache-line lookups of the fine levels, the kernel's bound
-// (800x800 render: field 81.9 -> 54.8 ms; pairing only the even-x corners
-// in one 8-byte load, as the encode kernel does, measured 11 % slower).
-// The fp16 features go through LDS (rows of 80 bytes: 16-byte
-// stores of four levels, 16-byte reads of lane group g's levels 4g..4g+3,
-// no bank conflicts) into the MLP's B-operand layout, four 16-sample tiles
-// per group; the SH coefficients go through LDS as in k_field_mlp.
+// halves the cache lines of the fine levels.
+// What bounds it: the vector-memory path and, beside it, the vector ALUs.
+// The levels run in rolled loops of two (16 unrolled bodies with three paths
+// each held so many uniform values that 190 of them went through spill lanes,
+// 2,700 vector instructions per group of 64 samples against 2,100), the
+// corner sums take v_fma_mix_f32 (corner_sum), and an incoherent level's
+// entries are fetched as aligned pairs (entry_pair).  Together, 800x800
+// render 44.4 -> 40.9 ms, three 1280x720 views over five cascades
+// 471 -> 373 ms.
+// The fp16 features go through LDS (rows of 80 bytes, 16-byte reads of lane
+// group g's levels 4g..4g+3) into the MLP's B-operand layout, four 16-sample
+// tiles per group; the SH coefficients go through LDS as in k_field_mlp.
 constexpr uint32_t kFeatPitch = 40u;  // halves per LDS feature row (80 bytes)
 template <typename TableT, bool kFromSamples>
 __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g, const TableT* __restrict__ table, const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, FieldInputs in, uint32_t n_cap,
@@ -233,6 +238,10 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
     load_density(sp, fd, lane);
     load_color(sp + NERF_EXT_DENSITY_PARAMS, fc, lane);
     half_t* F = feat[wv];
+    const uint32_t n_narrow = in.narrow_end;
+    uint32_t n_dense      = 0u;  // leading dense levels
+#pragma unroll
+    for (uint32_t l = 0; l < 16u; ++l) n_dense += g.dense[l] != 0u ? 1u : 0u;
     // Round r covers groups [r * W, (r + 1) * W) (W = all waves), XCD x
     // (workgroups b with b % 8 == x) taking the x-th eighth of it.
     const uint32_t groups  = (n + 63u) / 64u;
@@ -259,23 +268,32 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
         sh16(d, sh);
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) shl[wv][lane][j] = half4_t{to_half_rne(sh[4u * j]), to_half_rne(sh[4u * j + 1u]), to_half_rne(sh[4u * j + 2u]), to_half_rne(sh[4u * j + 3u])};
-        // Gather, four levels per 16-byte LDS store.
-#pragma unroll
-        for (uint32_t k = 0; k < 4u; ++k) {
-            half8_t h;
-#pragma unroll
-            for (uint32_t j = 0; j < 4u; ++j) {
-                const uint32_t l = 4u * k + j;
-                float a0 = 0.0f, a1 = 0.0f;
-                if (l < g.n_levels) {
-                    if (g.dense[l] != 0u) encode_level_xpair<TableT, false>(g, table, p, l, g.resolution[l], true, a0, a1);
-                    else encode_level_lanepair<TableT>(g, table, p, l, g.resolution[l], false, a0, a1);
-                }
-                h[2u * j]      = to_half_rne(a0);
-                h[2u * j + 1u] = to_half_rne(a1);
+        // Gather: rolled loops over the dense and the hashed levels (in that
+        // order: resolutions grow with the level), two levels at a time,
+        // features to LDS as they come.
+        auto put = [&](uint32_t l, float a0, float a1) { *reinterpret_cast<half2_t*>(F + lane * kFeatPitch + 2u * l) = half2_t{to_half_rne(a0), to_half_rne(a1)}; };
+        uint32_t l = 0u;
+        auto levels_to = [&](uint32_t end, auto level) {
+            for (; l + 2u <= end; l += 2u) {
+                float a0, a1, b0, b1;
+                level(l, a0, a1);
+                level(l + 1u, b0, b1);
+                put(l, a0, a1);
+                put(l + 1u, b0, b1);
             }
-            *reinterpret_cast<half8_t*>(F + lane * kFeatPitch + 8u * k) = h;
-            if (in.features_out && s < n) *reinterpret_cast<half8_t*>(in.features_out + (uint64_t)s * 32u + 8u * k) = h;
+            for (; l < end; ++l) {
+                float a0, a1;
+                level(l, a0, a1);
+                put(l, a0, a1);
+            }
+        };
+        levels_to(n_dense, [&](uint32_t k, float& a0, float& a1) { encode_level_xpair<TableT, false, kFromSamples>(g, table, p, k, g.resolution[k], true, a0, a1); });
+        levels_to(n_narrow, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFromSamples, false>(g, table, p, k, g.resolution[k], false, a0, a1); });
+        levels_to(16u, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFromSamples>(g, table, p, k, g.resolution[k], false, a0, a1); });
+        if (in.features_out && s < n) {
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) *reinterpret_cast<half8_t*>(in.features_out + (uint64_t)s * 32u + 8u * k) = *reinterpret_cast<const half8_t*>(F + lane * kFeatPitch + 8u * k);
         }
         __builtin_amdgcn_wave_barrier();  // LDS traffic of one wave completes in order
         float v[4];

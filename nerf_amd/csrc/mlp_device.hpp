@@ -198,7 +198,7 @@ __device__ __forceinline__ floatx4 color_mlp(const ColorFrags& f, const half8_t 
 }
 
 // Hash encoding of levels 4g..4g+3 of one point: features 8g..8g+7 as fp32.
-template <typename TableT>
+template <typename TableT, bool kFma = false>
 __device__ __forceinline__ void encode_quad(const GridParams& g, const TableT* __restrict__ table, const float p[3], uint32_t grp, float feat[8]) {
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j) {
@@ -214,7 +214,7 @@ __device__ __forceinline__ void encode_quad(const GridParams& g, const TableT* _
         // the lane groups of a wave hold both kinds at once, and the 8-byte
         // x-pair loads of encode_level_xpair ran both branches (measured 1.5x
         // slower than one load per corner).
-        if (level < g.n_levels) encode_level_lanepair(g, table, p, level, N, dn != 0u, a0, a1);
+        if (level < g.n_levels) encode_level_lanepair<TableT, kFma>(g, table, p, level, N, dn != 0u, a0, a1);
         feat[2u * j]      = a0;
         feat[2u * j + 1u] = a1;
     }
