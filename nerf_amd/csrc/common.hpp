@@ -404,6 +404,19 @@ __device__ __forceinline__ void encode_level_lanepair(const GridParams& g, const
     else corner_sum<kFma>(c, v, a0, a1);
 }
 
+// One level from its cell table (CellTables): the 8 corner entries of a cell
+// lie together in corner order, 32 bytes, fetched by two 16-byte loads.  Same
+// entries, weights and summation order as the other paths.
+template <bool kFma>
+__device__ __forceinline__ void encode_level_cell(const uint4* __restrict__ cells, const float p[3], uint32_t N, float& a0, float& a1) {
+    const LevelCell c  = level_cell(p, N);
+    const uint32_t off = 32u * ((c.i0[2] * N + c.i0[1]) * N + c.i0[0]);  // a level's table is below 4 GiB
+    const uint4* q     = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(cells) + off);
+    const uint4 lo = q[0], hi = q[1];
+    const uint32_t v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    corner_sum<kFma>(c, v, a0, a1);
+}
+
 // --------------------------------------------------------------- cameras
 struct Ray {
     float o[3];
@@ -459,6 +472,15 @@ __device__ __forceinline__ bool pixel_ray(const NerfExtCamera& c, uint32_t pix, 
 // field pass.
 __device__ __forceinline__ float render_alpha(float sigma, float dt) { return 1.0f - __expf(-(sigma * fmaxf(dt, 0.0f))); }
 
+// Levels [0, levels) of a table laid out cell by cell: cell (x, y, z) of
+// level l is entry first[l] + x + y N + z N^2, its 8 corners' fp16 pairs in
+// corner order (32 bytes).  Filled by build_cell_tables.
+struct CellTables {
+    uint4* data;  // two per cell
+    uint32_t levels;
+    uint32_t first[NERF_EXT_MAX_LEVELS];
+};
+
 struct FieldInputs {
     // Mode A: explicit positions [n][3] and directions [n][3].
     const float* positions;
@@ -500,6 +522,9 @@ struct FieldInputs {
     // level-split encode writes (each XCD whole lines of its levels) instead
     // of features_out, and the MLP pass reads.
     uint32_t* features_lm;
+    // Optional (fp16 table): the leading levels cell by cell (level-major
+    // kernel).
+    CellTables cells;
     // Hashed levels below this one are gathered by 4-byte loads (level-major
     // kernel; fp16 table).
     uint32_t narrow_end;
@@ -554,6 +579,8 @@ struct FieldWeights {
 // Level-split encode of a march sample stream: features [cap][32] fp16 rows,
 // or with lm, level-major fp16 pairs lm[level * cap + sample].
 hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const FieldInputs& in, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream);
+// Fills the cell tables of levels [0, t.levels) from the hash table (fp16).
+hipError_t build_cell_tables(const GridParams& g, const half_t* table, const CellTables& t, hipStream_t stream);
 // out4 [n] float4 (sigma, r, g, b).
 hipError_t launch_field(const GridParams& g, const void* table, const FieldWeights& w, const FieldInputs& in, uint32_t n, float4* out4, hipStream_t stream);
 // Density network only, on points or on fp16 features: out [n][16] = (exp(raw0), raw1..15).

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
     load_density(sp, fd, lane);
     load_color(sp + NERF_EXT_DENSITY_PARAMS, fc, lane);
     half_t* F = feat[wv];
-    const uint32_t n_narrow = in.narrow_end;
+    const uint32_t n_cell = in.cells.levels, n_narrow = in.narrow_end;
     uint32_t n_dense      = 0u;  // leading dense levels
 #pragma unroll
     for (uint32_t l = 0; l < 16u; ++l) n_dense += g.dense[l] != 0u ? 1u : 0u;
@@ -268,9 +268,9 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
         sh16(d, sh);
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) shl[wv][lane][j] = half4_t{to_half_rne(sh[4u * j]), to_half_rne(sh[4u * j + 1u]), to_half_rne(sh[4u * j + 2u]), to_half_rne(sh[4u * j + 3u])};
-        // Gather: rolled loops over the dense and the hashed levels (in that
-        // order: resolutions grow with the level), two levels at a time,
-        // features to LDS as they come.
+        // Gather: rolled loops over the cell-table, dense and hashed levels
+        // (in that order: resolutions grow with the level), two levels at a
+        // time, features to LDS as they come.
         auto put = [&](uint32_t l, float a0, float a1) { *reinterpret_cast<half2_t*>(F + lane * kFeatPitch + 2u * l) = half2_t{to_half_rne(a0), to_half_rne(a1)}; };
         uint32_t l = 0u;
         auto levels_to = [&](uint32_t end, auto level) {
@@ -287,6 +287,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
                 put(l, a0, a1);
             }
         };
+        levels_to(n_cell, [&](uint32_t k, float& a0, float& a1) { encode_level_cell<kFromSamples>(in.cells.data + 2ull * in.cells.first[k], p, g.resolution[k], a0, a1); });
         levels_to(n_dense, [&](uint32_t k, float& a0, float& a1) { encode_level_xpair<TableT, false, kFromSamples>(g, table, p, k, g.resolution[k], true, a0, a1); });
         levels_to(n_narrow, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFromSamples, false>(g, table, p, k, g.resolution[k], false, a0, a1); });
         levels_to(16u, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFromSamples>(g, table, p, k, g.resolution[k], false, a0, a1); });

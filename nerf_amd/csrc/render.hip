@@ -661,6 +661,7 @@ struct NerfExtRenderer {
     Buf<uint32_t> keep, koff;          // slots carried into the next round, their positions there
     Buf<unsigned long long> keep_total;
     Buf<unsigned long long> round_total;
+    Buf<uint4> cells;                  // cell tables of the leading levels
     Buf<nerf_hip::half8_t> ref_frags;           // reference-model weights in MFMA fragment order
     hipEvent_t ev[6] = {};
     hipEvent_t fev[2 * kMaxRounds] = {};
@@ -689,6 +690,7 @@ struct NerfExtRenderer {
         qlist.release();
         qray.release();
         round_total.release();
+        cells.release();
         for (hipEvent_t& e : fev)
             if (e) (void)hipEventDestroy(e);
         for (hipEvent_t& e : ev)
@@ -740,8 +742,9 @@ hipError_t scratch_address(void** out) {
 // few runs of entries, which 4-byte loads return in 5-16 cycles and 8-byte
 // loads in 16; on finer levels nearly every lane pair has a line of its own
 // (37 against 19 cycles, L1-resident).  800x800 over the unit box (spacing
-// 1/841): all levels narrow 42.3 ms, all wide 40.9 ms;
-// 3 x 1280x720 over five cascades (1/14200): narrow 373 ms, all wide 410 ms.
+// 1/841): all levels narrow 37.5 ms, narrow below resolution 405 35.9 ms;
+// 3 x 1280x720 over five cascades (1/14200): narrow 338 ms, all wide 359 ms,
+// the finest level alone wide 348 ms.
 uint32_t narrow_levels(const GridParams& g, const NerfExtCamera* cams, uint32_t views, const float lo[3], const float hi[3]) {
     const float extent = std::max({hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]});
     float spacing      = 0.0f;  // the widest view's, in box lengths
@@ -756,6 +759,38 @@ uint32_t narrow_levels(const GridParams& g, const NerfExtCamera* cams, uint32_t 
     uint32_t n = 0u;
     while (n < g.n_levels && (float)g.resolution[n] * spacing < 0.4f) ++n;
     return n;
+}
+
+// Cell tables of a render of up to `samples` samples: leading levels of an
+// fp16 table while a level has at most a sixteenth as many cells as the
+// render may have samples and all tables fit in 2 GiB.  Filling costs about
+// 6 ps per cell (41 M cells, 254 us) and a level's gather saves about 6 ps
+// per sample marched (800x800: 4.5 ms of 42 for ten levels and 370 M samples);
+// a third to a half of the possible samples are marched, and an early stop
+// leaves fewer.  Renders of fewer than 2^24 possible samples gain less than
+// the extra launch costs (100x75 at 256 steps: 299 -> 304 us).  Without
+// memory for the tables the render reads the hash table.
+constexpr uint64_t kCellMinSamples = 1ull << 24;
+constexpr uint64_t kCellMax        = 1ull << 26;  // cells of all tables (32 bytes each)
+constexpr uint32_t kCellMaxRes     = 511u;        // a level's table stays below 4 GiB (32-bit offsets)
+hipError_t plan_cells(NerfExtRenderer* R, const GridParams& g, const void* table, uint64_t samples, FieldInputs& in, hipStream_t st) {
+    in.cells.levels = 0u;
+    if (g.table_dtype != NERF_EXT_F16 || samples < kCellMinSamples) return hipSuccess;
+    uint64_t total = 0;
+    for (uint32_t l = 0; l < g.n_levels; ++l) {
+        const uint64_t N = g.resolution[l], cells = N * N * N;
+        if (N > kCellMaxRes || cells > samples / 16u || total + cells > kCellMax) break;
+        in.cells.first[l] = (uint32_t)total;
+        in.cells.levels   = l + 1u;
+        total += cells;
+    }
+    if (R->cells.reserve(2u * total) != hipSuccess) {
+        (void)hipGetLastError();
+        in.cells.levels = 0u;
+        return hipSuccess;
+    }
+    in.cells.data = R->cells.ptr;
+    return build_cell_tables(g, (const half_t*)table, in.cells, st);
 }
 
 }  // namespace
@@ -964,6 +999,7 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
     }
     if (!ref_model) {
         in.narrow_end = narrow_levels(g, d->cameras, d->view_count, occ.omin, occ.omax);
+        if (slots) NERF_HIP_TRY(plan_cells(R, g, d->model->table, (uint64_t)n_rays << slot_shift, in, st));
     }
     const float3 bg = make_float3(d->background[0], d->background[1], d->background[2]);
     // Rounds: the schedule's round ends 256, 512, 1024, ... until every
@@ -1153,6 +1189,7 @@ NERF_API NerfStatus nerf_ext_render_uniform(NerfExtRenderer* R, const NerfExtMod
     }
     if (!ref_model) {
         in.narrow_end = narrow_levels(g, cameras, view_count, aabb6, aabb6 + 3);
+        NERF_HIP_TRY(plan_cells(R, g, model->table, (uint64_t)n_rays * samples_per_ray, in, st));
     }
     const float3 bg = background3 ? make_float3(background3[0], background3[1], background3[2]) : make_float3(1.0f, 1.0f, 1.0f);
     for (uint32_t ray0 = 0; ray0 < n_rays; ray0 += chunk_rays) {

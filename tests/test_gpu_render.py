@@ -128,3 +128,25 @@ def test_render_in_chunks_matches_one_chunk():
     (a0, r0, c0, s0, h0), (a1, r1, c1, s1, h1) = outs
     assert np.array_equal(a0, a1) and np.array_equal(r0.view(np.uint32), r1.view(np.uint32)) and np.array_equal(c0, c1)
     assert s0 == s1 == int(c0.sum()) and h0 == h1 and s0 > 0
+
+
+@pytest.mark.parametrize("log2_t,finest,width,height", [(19, 0, 160, 110), (15, 0, 171, 103), (21, 4096, 160, 120)])
+def test_render_with_cell_tables_matches_hash_table(log2_t, finest, width, height):
+    # At least 2^24 possible samples: the default chunking gathers the leading
+    # levels from cell tables (dense and hashed ones: T = 2^15 hashes from
+    # resolution 42 on), an explicit sample budget reads the hash table.  Same
+    # entries, weights and sums, so the images are the same bit for bit.
+    assert (width * height) << 10 >= 1 << 24
+    announce(f"render {width}x{height} from cell tables, T=2^{log2_t} finest={finest}")
+    _, bits = _scene_setup()
+    desc = ext.grid_desc(log2_t, L.NERF_EXT_F16, finest=finest)
+    model = ext.Model.create(desc, seed=4, table_range=1.0)
+    cams = [ext.camera_orbit(0, 3, 1.32, CENTRE, width, height, 1111.0 * width / 800.0)]
+    occ = ext.occupancy_struct(bits, 128)
+    outs = []
+    for chunk in (0, 1 << 22):
+        rgb = DeviceArray((1, height, width, 3), np.float32)
+        rgba, _ = ext.Renderer().render(model, occ, cams, 1024, rgb=rgb, chunk_samples=chunk)
+        synchronize()
+        outs.append((rgba.numpy(), rgb.numpy().view(np.uint32)))
+    assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
