@@ -593,7 +593,9 @@ hipError_t launch_density(const GridParams& g, const void* table, const half_t* 
 // positions), out4 = (softplus sigma, sigmoid rgb), raw4 optional.
 constexpr uint32_t kRefFragments = 444u;
 hipError_t ref_pack_weights(const half_t* dparams, const half_t* cparams, half8_t* frags, hipStream_t stream);
-hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_t n, float4* out4, float4* raw4, hipStream_t stream);
+hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_t n, float4* out4, float4* raw4, hipStream_t stream, half_t* dens_out = nullptr);
+// Workgroups, and partials, of the weight-gradient kernels.
+uint32_t ref_grad_blocks(uint32_t np);
 // Training of the reference model (the trainer's stages).  Rows of the
 // neuron-major fp16 buffers (blocks of 32 samples) the backward writes per sample: every layer's
 // input (acts) and output delta (dlts); weight-gradient partials per chunk of
@@ -605,11 +607,10 @@ constexpr uint32_t kRefReduceBlocks = (kRefParams + 255u) / 256u;  // one parame
 constexpr uint32_t kRefMaxSamples = 1u << 20;  // per backward call: the buffers stay below 4 GiB (buffer-descriptor range)
 struct RefTrainLaunch {
     half8_t* frags;    // 64 x kRefFragments
-    half_t* acts;      // [kRefActRows][np]
-    half_t* dlts;      // [kRefDltRows][np]
-    float* partial;    // [chunks][kRefParams]
+    half_t* dens;      // [np][16] the forward's density outputs
+    half_t* deltas;    // [np][16] their deltas
+    float* partial;    // [ref_grad_blocks(np)][kRefParams]
     uint32_t np;       // sample capacity rounded up to 64
-    uint32_t chunks;   // ceil(np / kRefDwChunk)
     uint32_t max_rays;
 };
 // Composite forward/backward with the reference's loss on the trainer's

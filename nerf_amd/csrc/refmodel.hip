@@ -171,6 +171,21 @@ __device__ __forceinline__ half8_t frag_load(const FragSrc& S, uint32_t f) {
 // replace four 2-byte stores (a quarter of the store instructions, each a
 // full wave of lane addresses for the address path).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x2 quad_transpose(half4_t h) {
+    constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E;  // quad_perm [1, 0, 3, 2] and [2, 3, 0, 1]
+    const uint32_t j = threadIdx.x & 3u;
+    const uint32_t a = __builtin_bit_cast(uint32_t, half2_t{h[0], h[1]}), b = __builtin_bit_cast(uint32_t, half2_t{h[2], h[3]});
+    const uint32_t a1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)a, kSwap1, 0xf, 0xf, false);
+    const uint32_t b1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, kSwap1, 0xf, 0xf, false);
+    // Even lanes: (own, next) of their first row; odd lanes: (previous,
+    // own) of their second row.
+    const uint32_t sel = (j & 1u) ? 0x03020706u : 0x05040100u;
+    const uint32_t c = __builtin_amdgcn_perm(a1, a, sel), d = __builtin_amdgcn_perm(b1, b, sel);
+    const uint32_t c2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)c, kSwap2, 0xf, 0xf, false);
+    const uint32_t d2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)d, kSwap2, 0xf, 0xf, false);
+    const bool first  = j < 2u;
+    return u32x2{first ? c : d2, first ? c2 : d};
+}
 // One block of a layer's rows is one contiguous run for k_ref_dw (rows at a
 // stride of the sample count, 64 bytes per row and step, read back more
 // slowly), and a group's stores land in two blocks.  A wave's group of 64 samples is blocks blk and blk + 1; tile t (16
@@ -186,21 +201,7 @@ struct RowStore {
     __device__ __forceinline__ void put(uint32_t row_u, uint32_t t, half_t v) const {
         __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rsrc, vbase + 32u * (t & 1u), soff(row_u, t), 0);
     }
-    __device__ __forceinline__ void put_quad(uint32_t row_u, uint32_t t, half4_t h) const {
-        constexpr int kSwap1 = 0xB1, kSwap2 = 0x4E;  // quad_perm [1, 0, 3, 2] and [2, 3, 0, 1]
-        const uint32_t j = threadIdx.x & 3u;
-        const uint32_t a = __builtin_bit_cast(uint32_t, half2_t{h[0], h[1]}), b = __builtin_bit_cast(uint32_t, half2_t{h[2], h[3]});
-        const uint32_t a1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)a, kSwap1, 0xf, 0xf, false);
-        const uint32_t b1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, kSwap1, 0xf, 0xf, false);
-        // Even lanes: (own, next) of their first row; odd lanes: (previous,
-        // own) of their second row.
-        const uint32_t sel = (j & 1u) ? 0x03020706u : 0x05040100u;
-        const uint32_t c = __builtin_amdgcn_perm(a1, a, sel), d = __builtin_amdgcn_perm(b1, b, sel);
-        const uint32_t c2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)c, kSwap2, 0xf, 0xf, false);
-        const uint32_t d2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)d, kSwap2, 0xf, 0xf, false);
-        const bool first  = j < 2u;
-        __builtin_amdgcn_raw_buffer_store_b64(u32x2{first ? c : d2, first ? c2 : d}, rsrc, vquad + 32u * (t & 1u), soff(row_u, t), 0);
-    }
+    __device__ __forceinline__ void put_quad(uint32_t row_u, uint32_t t, half4_t h) const { __builtin_amdgcn_raw_buffer_store_b64(quad_transpose(h), rsrc, vquad + 32u * (t & 1u), soff(row_u, t), 0); }
     __device__ __forceinline__ half_t get(uint32_t row_u, uint32_t t) const {
         return __builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(rsrc, vbase + 32u * (t & 1u), soff(row_u, t), 0));
     }
@@ -438,8 +439,12 @@ __device__ __forceinline__ void freq_row(const float v[3], uint32_t levels, half
     w[1u + 3u * levels] = pack(carry, (half_t)0.0f);
 }
 
-template <bool kFromSamples>
-__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ref_field(const half8_t* __restrict__ frags, FieldInputs in, uint32_t n_cap, float4* __restrict__ out, float4* __restrict__ raw_out) {
+// With dens_out, the density network's 16 fp16 outputs also go to
+// dens_out[sample][16] (the weight gradients' colour pass starts from them);
+// kDensityOnly: nothing else is computed.
+template <bool kFromSamples, bool kDensityOnly = false>
+__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ref_field(const half8_t* __restrict__ frags, FieldInputs in, uint32_t n_cap, float4* __restrict__ out, float4* __restrict__ raw_out,
+                                                                                                         half_t* __restrict__ dens_out) {
     const uint32_t n = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
     __shared__ __align__(16) half_t rows[kBlockWaves][64 * kRefPitch];
     const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, s16 = lane & 15u, wv = wave_index();
@@ -474,9 +479,11 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2
             half_t* row = R + lane * kRefPitch;
             freq_row(p, 10u, row);
             row[63] = (half_t)0.0f;
-            freq_row(d, 4u, row + 64u);
+            if constexpr (!kDensityOnly) {
+                freq_row(d, 4u, row + 64u);
 #pragma unroll
-            for (uint32_t k = 64u + 27u; k < 96u; ++k) row[k] = (half_t)0.0f;
+                for (uint32_t k = 64u + 27u; k < 96u; ++k) row[k] = (half_t)0.0f;
+            }
         }
         __builtin_amdgcn_wave_barrier();  // LDS traffic of one wave completes in order
         half8_t x[4][4], y[4][4];
@@ -495,6 +502,17 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2
         ref_hidden<4>(S, kRefLayers[4].frag0, x, y);
         floatx4 dens[4];
         ref_output(S, kRefLayers[5].frag0, y, dens);
+        if (kDensityOnly || dens_out) {
+#pragma unroll
+            for (uint32_t t = 0; t < 4u; ++t) {
+                const uint32_t st = gi * 64u + 16u * t + s16;
+                if (st < n) *reinterpret_cast<half4_t*>(dens_out + (uint64_t)st * 16u + 4u * g) = __builtin_convertvector(dens[t], half4_t);
+            }
+        }
+        if constexpr (kDensityOnly) {
+            __builtin_amdgcn_wave_barrier();  // the next group rewrites the rows
+            continue;
+        }
         // Colour input: raw density outputs 4g..4g+3 (fp16) and direction
         // encoding 4g..4g+3; then direction encoding 16 + 8g .. + 7.
 #pragma unroll
@@ -547,15 +565,12 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2
 // capped, it spills 77 VGPRs to scratch and the pass still runs faster
 // (503 -> 476 us per 2^18 samples): with one wave nothing hides the weight
 // fragment, LDS and MFMA latencies of the layer chain.
-template <bool kFromSamples>
-__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ref_backward(const half8_t* __restrict__ frags, FieldInputs in, uint32_t n_cap, const float4* __restrict__ draw, float loss_scale, half_t* __restrict__ acts,
+__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ref_backward(const half8_t* __restrict__ frags, FieldInputs in, uint32_t n, const float4* __restrict__ draw, float loss_scale, half_t* __restrict__ acts,
                                                                 half_t* __restrict__ dlts, uint32_t np) {
     __shared__ __align__(16) half_t rows[kBlockWaves][64 * kRefPitch];
     const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, s16 = lane & 15u, wv = wave_index();
     half_t* R       = rows[wv];
     const FragSrc S = frag_src(frags, lane);
-    // Samples: n_cap, or the count on the device (the trainer's) clamped to it.
-    const uint32_t n      = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
     const uint32_t groups = (n + 63u) / 64u;
     const __amdgpu_buffer_rsrc_t ra = row_rsrc(acts, kActRows, np), rd = row_rsrc(dlts, kDltRows, np);
     for (uint32_t gi = blockIdx.x * kBlockWaves + wv; gi < groups; gi += gridDim.x * kBlockWaves) {
@@ -567,22 +582,10 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2
         {
             const uint32_t q = min(s0 + lane, n - 1u);
             float p[3], d[3];
-            if constexpr (kFromSamples) {
-                const float2 td  = in.samples[q];
-                const uint32_t r = in.sample_ray[q];
-                const float4 ro = in.rays[2ull * r], rd = in.rays[2ull * r + 1ull];
-                d[0] = rd.x;
-                d[1] = rd.y;
-                d[2] = rd.z;
-                p[0] = ro.x + td.x * rd.x;
-                p[1] = ro.y + td.x * rd.y;
-                p[2] = ro.z + td.x * rd.z;
-            } else {
 #pragma unroll
-                for (uint32_t a = 0; a < 3u; ++a) {
-                    p[a] = in.positions[3ull * q + a];
-                    d[a] = in.directions[3ull * q + a];
-                }
+            for (uint32_t a = 0; a < 3u; ++a) {
+                p[a] = in.positions[3ull * q + a];
+                d[a] = in.directions[3ull * q + a];
             }
             half_t* row = R + lane * kRefPitch;
             freq_row(p, 10u, row);
@@ -694,11 +697,8 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(2
 constexpr uint32_t kRefDwRows  = 256u;  // largest n_out + n_in
 constexpr uint32_t kRefDwStage = kRefDwRows * 64u;  // bytes per step of 32 samples
 
-// np is the row pitch of the buffers; with n_dev the rows hold
-// ceil(min(*n_dev, np) / 64) groups (the rest is stale) and later chunks
-// write zero partials.
-__global__ __launch_bounds__(kBlockThreads) void k_ref_dw(const half_t* __restrict__ acts, const half_t* __restrict__ dlts, uint32_t np, uint32_t chunk, uint32_t chunks, float* __restrict__ partial,
-                                                          const uint32_t* __restrict__ n_dev) {
+// np is the row pitch of the buffers.
+__global__ __launch_bounds__(kBlockThreads) void k_ref_dw(const half_t* __restrict__ acts, const half_t* __restrict__ dlts, uint32_t np, uint32_t chunk, uint32_t chunks, float* __restrict__ partial) {
     __shared__ __align__(16) unsigned char stage[2][kRefDwStage];
     // The wave index stays a vector value here: as a scalar (wave_index) the
     // pass took 393 us instead of 300 per 2^18 samples.
@@ -723,8 +723,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_ref_dw(const half_t* __restri
         nc = cb_all / 4u;
         c0 = wv * nc;
     }
-    const uint32_t n_used  = n_dev ? (min(*n_dev, np) + 63u) / 64u * 64u : np;
-    const uint32_t k_begin = min(kc * chunk, n_used), k_end = min(n_used, kc * chunk + chunk);
+    const uint32_t k_begin = kc * chunk, k_end = min(np, k_begin + chunk);
     // Staging: thread t copies 16 bytes (8 samples) of row t / 4 + 64 j.
     const uint32_t srow = threadIdx.x >> 2, spart = threadIdx.x & 3u;
     // Row r of step k0 (a whole 32-sample block): the layer's delta rows, then
@@ -848,6 +847,489 @@ __global__ __launch_bounds__(256) void k_ref_dw_reduce(const float* __restrict__
         const double b = ((wsq[0] + wsq[1]) + wsq[2]) + wsq[3];
         norm[blockIdx.x] = (wbad[0] | wbad[1] | wbad[2] | wbad[3]) ? -1.0 - b : b;
     }
+}
+
+// ------------------------------------------------- fused weight gradients
+// The backward without rows in memory: two kernels, one per network, whose
+// workgroups (one per CU, 8 waves, 64 samples at a time) recompute the
+// forward, back-propagate and multiply the weight gradients from LDS, and
+// keep the network's whole gradient in registers until their last group.
+// Storing every layer's rows for a separate product (k_ref_backward and
+// k_ref_dw, 4.4 KB written and read per sample) was bound by that traffic:
+// 640 us per 2^18 samples; the second forward of the density network costs a
+// fifth more matrix work instead.
+//
+//   k_ref_grad_color    colour forward (from the density outputs that
+//                       k_ref_field left) and backward; writes the density
+//                       outputs' deltas [sample][16] (geometry and sigma) for
+//   k_ref_grad_density  density forward and backward.
+//
+// A layer's 128 outputs are split over the waves, 16 neurons x 64 samples
+// each, so a group reads each weight fragment once; activations pass between
+// waves in LDS, double-buffered, one barrier per layer:
+//   * fragment order (16 KiB): the next product's B operands, 16-byte slots
+//     [k-block][tile][lane];
+//   * rows (neuron-major, 128 bytes per neuron: 64 samples): the operands of
+//     the weight gradients, samples on the reduction axis.  The 16-byte
+//     chunks of a row are XORed with the row's low bits, so that the 16 rows
+//     of an operand read fall on distinct banks.
+// All 75,776 (40,960) gradients are MFMA accumulators: per 128 x 128 layer a
+// wave owns 64 x 32.  The register budget is that of two waves per SIMD.
+constexpr uint32_t kGradThreads = 512u;
+constexpr uint32_t kGradFrag    = 16384u;  // bytes of one fragment-order buffer
+constexpr uint32_t kRowBytes    = 128u;
+constexpr uint32_t kGradDensityRows = 64u + 5u * 128u, kGradColorRows = 48u + 3u * 128u;
+constexpr uint32_t kGradDensityLds  = kGradDensityRows * kRowBytes + 4u * kGradFrag + 16u * kRowBytes;
+constexpr uint32_t kGradColorLds    = kGradColorRows * kRowBytes + 4u * kGradFrag + 16u * kRowBytes + kGradFrag / 2u;
+static_assert(kGradDensityLds <= 160u * 1024u && kGradColorLds <= 160u * 1024u, "LDS of one workgroup");
+
+typedef unsigned char lds_byte;
+
+// One value of neuron k, sample s, in rows.
+__device__ __forceinline__ void row_put(lds_byte* rows, uint32_t k, uint32_t s, half_t v) { *reinterpret_cast<half_t*>(rows + k * kRowBytes + (((s >> 3) ^ (k & 7u)) << 4) + (s & 7u) * 2u) = v; }
+// A lane's offsets into those layouts, for one map of the LDS (kDrow, kFrag:
+// where the delta rows and the fragment buffers start; input rows start at 0).
+// A wave's share is in the offset, so that what remains of an address is a
+// constant that fits the instruction (below 64 KiB).  The offsets are made
+// opaque once per group: the compiler would otherwise compute every access'
+// address before the loop and keep them all in registers.
+struct GradLane {
+    uint32_t quad[4];  // per tile: the 8 bytes of the wave's row block that the lane holds after the quad transpose
+    uint32_t in[2];    // per 32 samples: input operand of the wave's first column block of a 32-column share
+    uint32_t dlt[2];   // delta operand of its first row block, in the delta rows
+    uint32_t frag;     // the lane's slot of the first fragment buffer
+    uint32_t fragw;    // the wave's row block in it
+    template <uint32_t kDrow, uint32_t kFrag>
+    __device__ __forceinline__ void init(uint32_t lane, uint32_t wv) {
+        const uint32_t g = lane >> 4, j = lane & 3u, k = (lane & 15u) >> 2, row = 4u * g + j;
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) quad[t] = (16u * wv + row) * kRowBytes + (((2u * t + (k >> 1)) ^ (row & 7u)) << 4) + (k & 1u) * 8u;
+#pragma unroll
+        for (uint32_t ks = 0; ks < 2u; ++ks) {
+            const uint32_t op = (lane & 15u) * kRowBytes + (((4u * ks + g) ^ (lane & 7u)) << 4);
+            in[ks]  = op + 32u * kRowBytes * (wv & 3u);
+            dlt[ks] = op + 64u * kRowBytes * (wv >> 2) + kDrow;
+        }
+        frag  = lane * 16u + kFrag;
+        fragw = (wv >> 1) * 4096u + lane * 16u + (wv & 1u) * 8u + kFrag;
+    }
+    __device__ __forceinline__ void hide() {
+        asm volatile("" : "+v"(quad[0]), "+v"(quad[1]), "+v"(quad[2]), "+v"(quad[3]), "+v"(in[0]), "+v"(in[1]), "+v"(dlt[0]), "+v"(dlt[1]), "+v"(frag), "+v"(fragw));
+    }
+};
+extern __shared__ __align__(16) lds_byte grad_lds[];
+// A lane's results of one tile of its wave's row block (neurons 16 wv + 4 g +
+// e, sample 16 t + s16) to the rows at byte `rows`: the quad transpose of
+// RowStore::put_quad, then one 8-byte store.
+__device__ __forceinline__ void row_put_quad(uint32_t rows, const GradLane& L, uint32_t t, half4_t h) { *reinterpret_cast<u32x2*>(grad_lds + (L.quad[t] + rows)) = quad_transpose(h); }
+// MFMA operand of 16 rows, 32 samples: lane (g, i) holds row i, samples 8 g
+// .. + 7; off = one of the lane's operand offsets.
+__device__ __forceinline__ half8_t row_operand(uint32_t off) { return *reinterpret_cast<const half8_t*>(grad_lds + off); }
+// Operand of k-block q, tile t in fragment buffer `buf` (0, 1; 2: the colour
+// input's).
+__device__ __forceinline__ half8_t frag_read(uint32_t buf, const GradLane& L, uint32_t q, uint32_t t) { return *reinterpret_cast<const half8_t*>(grad_lds + (L.frag + buf * kGradFrag + (q * 4u + t) * 1024u)); }
+
+// A operands of row block r of a layer whose fragments start at f0.
+template <uint32_t KB>
+__device__ __forceinline__ void grad_weights(const FragSrc& S, uint32_t f0, uint32_t r, half8_t (&a)[KB]) {
+#pragma unroll
+    for (uint32_t q = 0; q < KB; ++q) a[q] = frag_load(S, f0 + r * KB + q);
+}
+
+// One row block times the group's four tiles.
+template <uint32_t KB>
+__device__ __forceinline__ void grad_product(const half8_t (&a)[KB], uint32_t in, const GradLane& L, floatx4 (&acc)[4]) {
+#pragma unroll
+    for (uint32_t t = 0; t < 4u; ++t) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    half8_t b[2][4];
+#pragma unroll
+    for (uint32_t t = 0; t < 4u; ++t) b[0][t] = frag_read(in, L, 0u, t);
+#pragma unroll
+    for (uint32_t q = 0; q < KB; ++q) {
+        // The next k-block's operands are requested before this one's
+        // products (left alone the scheduler waits for each operand alone).
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t)
+            if (q + 1u < KB) b[(q + 1u) & 1u][t] = frag_read(in, L, q + 1u, t);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) acc[t] = mfma16x16x32(a[q], b[q & 1u][t], acc[t]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Forward results of the wave's row block: ReLU, fp16, to the next product's operands
+// and (kRows) to rows; returns the ReLU mask (bit 4 t + e).
+template <bool kFrag, bool kRows>
+__device__ __forceinline__ uint32_t grad_emit(const floatx4 (&acc)[4], const GradLane& L, uint32_t out, uint32_t rows) {
+    uint32_t mask = 0u;
+#pragma unroll
+    for (uint32_t t = 0; t < 4u; ++t) {
+        const half4_t h = relu_half4(acc[t]);
+        if constexpr (kFrag) *reinterpret_cast<half4_t*>(grad_lds + (L.fragw + out * kGradFrag + 1024u * t)) = h;
+        if constexpr (kRows) {
+            row_put_quad(rows, L, t, h);
+            mask |= relu_bits(h) << (4u * t);
+        }
+    }
+    return mask;
+}
+
+// Backward results of row block r: zero where the forward's ReLU cleared the
+// neuron, fp16, to the next product's operands and to the delta rows.
+template <bool kFrag>
+__device__ __forceinline__ void grad_emit_delta(const floatx4 (&acc)[4], uint32_t mask, const GradLane& L, uint32_t out, uint32_t rows) {
+#pragma unroll
+    for (uint32_t t = 0; t < 4u; ++t) {
+        floatx4 v = acc[t];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) {
+            const float x = v[e];
+            v[e]          = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & (uint32_t)((int32_t)(mask << (31u - (4u * t + e))) >> 31));
+        }
+        const half4_t h = __builtin_convertvector(v, half4_t);
+        if constexpr (kFrag) *reinterpret_cast<half4_t*>(grad_lds + (L.fragw + out * kGradFrag + 1024u * t)) = h;
+        row_put_quad(rows, L, t, h);
+    }
+}
+
+// The fences keep the scheduler from gathering the operands of several
+// products at once, which spills the accumulators.
+// dW += delta rows x input rows over the group's 64 samples: the four row
+// blocks from delta + delta0, the CB column blocks from input + input0.
+template <uint32_t CB>
+__device__ __forceinline__ void grad_dw(floatx4 (&w)[4][CB], const uint32_t (&delta)[2], uint32_t delta0, const uint32_t (&input)[2], uint32_t input0) {
+    __builtin_amdgcn_sched_barrier(0);
+    half8_t fa[2][4], fb[2][CB];
+    auto fetch = [&](uint32_t ks) {
+#pragma unroll
+        for (uint32_t c = 0; c < CB; ++c) fb[ks][c] = row_operand(input[ks] + (input0 + 16u * c * kRowBytes));
+#pragma unroll
+        for (uint32_t r = 0; r < 4u; ++r) fa[ks][r] = row_operand(delta[ks] + (delta0 + 16u * r * kRowBytes));
+    };
+    fetch(0u);
+#pragma unroll
+    for (uint32_t ks = 0; ks < 2u; ++ks) {
+        if (ks == 0u) fetch(1u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t r = 0; r < 4u; ++r)
+#pragma unroll
+            for (uint32_t c = 0; c < CB; ++c) w[r][c] = mfma16x16x32(fa[ks][r], fb[ks][c], w[r][c]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <uint32_t CB>
+__device__ __forceinline__ void grad_dw_zero(floatx4 (&w)[4][CB]) {
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; ++r)
+#pragma unroll
+        for (uint32_t c = 0; c < CB; ++c) w[r][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+}
+template <uint32_t CB>
+__device__ __forceinline__ void grad_dw_store(const floatx4 (&w)[4][CB], float* dst, uint32_t n_in, uint32_t r0, uint32_t c0, uint32_t lane) {
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; ++r)
+#pragma unroll
+        for (uint32_t c = 0; c < CB; ++c)
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) dst[(16u * (r0 + r) + 4u * (lane >> 4) + e) * n_in + 16u * (c0 + c) + (lane & 15u)] = w[r][c][e];
+}
+// The 16-output layers: one row block, one column block.
+__device__ __forceinline__ void grad_dw_out(floatx4& w, const uint32_t (&delta)[2], uint32_t delta0, const uint32_t (&input)[2], uint32_t input0) {
+#pragma unroll
+    for (uint32_t ks = 0; ks < 2u; ++ks) w = mfma16x16x32(row_operand(delta[ks] + delta0), row_operand(input[ks] + input0), w);
+    __builtin_amdgcn_sched_barrier(0);
+}
+// Column block wv of the layer, the output deltas at byte `out`, its input
+// rows at `input`.
+__device__ __forceinline__ void grad_dw_output(floatx4& w, const GradLane& L, uint32_t out, uint32_t input, uint32_t wv) {
+    const uint32_t c = 32u * kRowBytes * (wv & 3u);  // the share L.in holds
+    const uint32_t op[2] = {L.in[0] - c, L.in[1] - c}, in[2] = {op[0] + 16u * kRowBytes * wv, op[1] + 16u * kRowBytes * wv};
+    grad_dw_out(w, op, out, in, input);
+}
+__device__ __forceinline__ void grad_dw_out_store(const floatx4& w, float* dst, uint32_t c, uint32_t lane) {
+#pragma unroll
+    for (uint32_t e = 0; e < 4u; ++e) dst[(4u * (lane >> 4) + e) * 128u + 16u * c + (lane & 15u)] = w[e];
+}
+
+template <bool kFromSamples>
+__device__ __forceinline__ void grad_point(const FieldInputs& in, uint32_t q, float p[3], float d[3]) {
+    if constexpr (kFromSamples) {
+        const float2 td = in.samples[q];
+        const uint32_t r = in.sample_ray[q];
+        const float4 ro = in.rays[2ull * r], rd = in.rays[2ull * r + 1ull];
+        d[0] = rd.x;
+        d[1] = rd.y;
+        d[2] = rd.z;
+        p[0] = ro.x + td.x * rd.x;
+        p[1] = ro.y + td.x * rd.y;
+        p[2] = ro.z + td.x * rd.z;
+    } else {
+#pragma unroll
+        for (uint32_t a = 0; a < 3u; ++a) {
+            p[a] = in.positions[3ull * q + a];
+            d[a] = in.directions[3ull * q + a];
+        }
+    }
+}
+
+// Frequency encoding of the group's 64 points (lane = sample), the sincos
+// pairs dealt over the waves; emit(feature, value) for each of the 3 +
+// 6 kLevels features once per group.
+template <uint32_t kLevels, typename Emit>
+__device__ __forceinline__ void grad_encode(const float v[3], uint32_t wv, Emit emit) {
+#pragma unroll 1
+    for (uint32_t pair = wv; pair < 3u * kLevels; pair += 8u) {  // uniform
+        const uint32_t l = pair / 3u, a = pair - 3u * l;
+        float s, c;
+        freq_sincos((a == 0u ? v[0] : a == 1u ? v[1] : v[2]) * (float)(1u << l), s, c);
+        emit(3u + 6u * l + a, to_half_rne(s));
+        emit(6u + 6u * l + a, to_half_rne(c));
+    }
+    if (wv == 6u) {
+#pragma unroll
+        for (uint32_t a = 0; a < 3u; ++a) emit(a, to_half_rne(v[a]));
+    }
+}
+// Feature k of a 64-wide input (identity k-map) in fragment order.
+__device__ __forceinline__ void frag_put_identity(lds_byte* f, uint32_t k, uint32_t s, half_t v) {
+    *reinterpret_cast<half_t*>(f + (((k >> 5) * 4u + (s >> 4)) * 64u + ((k >> 3) & 3u) * 16u + (s & 15u)) * 16u + (k & 7u) * 2u) = v;
+}
+// Direction feature d of the colour input in fragment order (ref_column).
+__device__ __forceinline__ void frag_put_direction(lds_byte* f, uint32_t d, uint32_t s, half_t v) {
+    const uint32_t q = d < 16u ? 0u : 1u, x = d < 16u ? d : d - 16u;
+    const uint32_t g = d < 16u ? x >> 2 : x >> 3, j = d < 16u ? 4u + (x & 3u) : x & 7u;
+    *reinterpret_cast<half_t*>(f + ((q * 4u + (s >> 4)) * 64u + g * 16u + (s & 15u)) * 16u + j * 2u) = v;
+}
+
+template <bool kFromSamples>
+__global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ref_grad_color(const half8_t* __restrict__ frags, FieldInputs in, uint32_t n_cap, const half_t* __restrict__ dens, const float4* __restrict__ draw, float loss_scale,
+                                                                                                            half_t* __restrict__ deltas, float* __restrict__ partial) {
+    constexpr uint32_t kLayer = 128u * kRowBytes;
+    constexpr uint32_t kHid = 0u;                           // 3 x 128 rows: the inputs of layers 7, 8, 9
+    constexpr uint32_t kCin = kHid + 3u * kLayer;           // 48 rows: the colour input
+    constexpr uint32_t kOut = kCin + 48u * kRowBytes;       // 16 rows: output deltas
+    constexpr uint32_t kDrow = kOut + 16u * kRowBytes;      // two buffers of 128 delta rows
+    constexpr uint32_t kFragAt = kDrow + 2u * kLayer;       // two fragment buffers, and the colour input's two k-blocks
+    static_assert(kFragAt + 2u * kGradFrag + kGradFrag / 2u == kGradColorLds, "LDS map");
+    lds_byte* const cin = grad_lds + kCin;
+    lds_byte* const dout = grad_lds + kOut;
+    lds_byte* const dfrag = grad_lds + kFragAt + 2u * kGradFrag;
+    const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, s16 = lane & 15u, wv = wave_index(), wr = wv >> 2, wc = wv & 3u;
+    GradLane L;
+    L.template init<kDrow, kFragAt>(lane, wv);
+    const FragSrc S       = frag_src(frags, lane);
+    const uint32_t n      = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
+    const uint32_t groups = (n + 63u) / 64u;
+    // Slots that no group writes (padding columns and output rows) are zero.
+    for (uint32_t i = threadIdx.x; i < (48u + 16u) * kRowBytes / 16u; i += kGradThreads) reinterpret_cast<uint4*>(cin)[i] = make_uint4(0u, 0u, 0u, 0u);  // and dout
+    for (uint32_t i = threadIdx.x; i < kGradFrag / 2u / 16u; i += kGradThreads) reinterpret_cast<uint4*>(dfrag)[i] = make_uint4(0u, 0u, 0u, 0u);
+    floatx4 w6[4][1], w7[4][2], w8[4][2], w9 = {0.0f, 0.0f, 0.0f, 0.0f};
+    grad_dw_zero(w6);
+    grad_dw_zero(w7);
+    grad_dw_zero(w8);
+    for (uint32_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+        const uint32_t s0 = gi * 64u;
+        L.hide();
+        half8_t a2[2], a4[4], a1[1];
+        floatx4 acc[4];
+        grad_weights(S, kRefLayers[6].frag0, wv, a2);
+        __syncthreads();  // the previous group's readers are done (and the zero fill)
+        {
+            float p[3], d[3];
+            grad_point<kFromSamples>(in, min(s0 + lane, n - 1u), p, d);
+            grad_encode<4u>(d, wv, [&](uint32_t k, half_t v) {
+                frag_put_direction(dfrag, k, lane, v);
+                row_put(cin, 15u + k, lane, v);
+            });
+        }
+        // The output deltas: lane group 0's four of each tile as operands, and
+        // the three used rows.
+        half8_t d9[4];
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) {
+            const uint32_t st = s0 + 16u * t + s16;
+            const float4 dr   = g == 0u && st < n ? draw[st] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            d9[t]             = half8_t{to_half_rne(loss_scale * dr.y), to_half_rne(loss_scale * dr.z), to_half_rne(loss_scale * dr.w), 0, 0, 0, 0, 0};
+            if (g == 0u && t == wc && wr == 0u) {
+#pragma unroll
+                for (uint32_t e = 0; e < 3u; ++e) row_put(dout, e, 16u * t + s16, d9[t][e]);
+            }
+        }
+        // Density outputs: tile wc by waves 4..7, into the colour input.
+        if (wr == 1u) {
+            const half4_t h = *reinterpret_cast<const half4_t*>(dens + (uint64_t)min(s0 + 16u * wc + s16, n - 1u) * 16u + 4u * g);
+            *reinterpret_cast<half4_t*>(dfrag + 1024u * wc + 16u * lane) = h;
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e)
+                if (4u * g + e >= 1u) row_put(cin, 4u * g + e - 1u, 16u * wc + s16, h[e]);
+        }
+        __syncthreads();
+        // Each step: the product, the request for the next step's weights
+        // (in flight across the rest of the step), its results.
+        grad_product(a2, 2u, L, acc);
+        grad_weights(S, kRefLayers[7].frag0, wv, a4);
+        const uint32_t m6 = grad_emit<true, true>(acc, L, 0u, kHid);
+        __syncthreads();
+        grad_product(a4, 0u, L, acc);
+        grad_weights(S, kRefLayers[8].frag0, wv, a4);
+        const uint32_t m7 = grad_emit<true, true>(acc, L, 1u, kHid + kLayer);
+        grad_weights(S, kRefT[0].frag0, wv, a1);
+        __syncthreads();
+        grad_product(a4, 1u, L, acc);
+        grad_weights(S, kRefT[1].frag0, wv, a4);
+        const uint32_t m8 = grad_emit<false, true>(acc, L, 0u, kHid + 2u * kLayer);
+        // delta of layer 8's outputs (needs no other wave's results).
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) acc[t] = mfma16x16x32(a1[0], d9[t], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+        grad_emit_delta<true>(acc, m8, L, 0u, kDrow);
+        __syncthreads();
+        grad_product(a4, 0u, L, acc);
+        grad_weights(S, kRefT[2].frag0, wv, a4);
+        grad_emit_delta<true>(acc, m7, L, 1u, kDrow + kLayer);
+        grad_dw_output(w9, L, kOut, kHid + 2u * kLayer, wv);
+        grad_dw(w8, L.dlt, 0u, L.in, kHid + kLayer);
+        __syncthreads();
+        grad_product(a4, 1u, L, acc);
+        grad_weights(S, kRefT[3].frag0, 0u, a4);
+        grad_emit_delta<true>(acc, m6, L, 0u, kDrow);
+        grad_dw(w7, L.dlt, kLayer, L.in, kHid);
+        __syncthreads();
+        if (wc < 3u) {
+            const uint32_t op[2] = {L.in[0] - 16u * kRowBytes * wc, L.in[1] - 16u * kRowBytes * wc};  // 16 columns per wave
+            grad_dw(w6, L.dlt, 0u, op, kCin);
+        }
+        if (wr == 1u) {  // density output deltas of tile wc
+            floatx4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; ++q) o = mfma16x16x32(a4[q], frag_read(0u, L, q, wc), o);
+            const uint32_t st = s0 + 16u * wc + s16;
+            half4_t h         = half4_t{to_half_rne(o[0]), to_half_rne(o[1]), to_half_rne(o[2]), to_half_rne(o[3])};
+            if (g == 0u) h[0] = to_half_rne(loss_scale * (st < n ? draw[st].x : 0.0f));
+            *reinterpret_cast<half4_t*>(deltas + (uint64_t)st * 16u + 4u * g) = h;
+        }
+    }
+    float* dst = partial + (uint64_t)blockIdx.x * (kRefDensityParams + kRefColorParams) + kRefDensityParams;
+    if (wc < 3u) grad_dw_store(w6, dst + kRefLayers[6].w_off, 48u, 4u * wr, wc, lane);
+    grad_dw_store(w7, dst + kRefLayers[7].w_off, 128u, 4u * wr, 2u * wc, lane);
+    grad_dw_store(w8, dst + kRefLayers[8].w_off, 128u, 4u * wr, 2u * wc, lane);
+    grad_dw_out_store(w9, dst + kRefLayers[9].w_off, wv, lane);
+}
+
+template <bool kFromSamples>
+__global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_ref_grad_density(const half8_t* __restrict__ frags, FieldInputs in, uint32_t n_cap, const half_t* __restrict__ deltas,
+                                                                                                              float* __restrict__ partial) {
+    constexpr uint32_t kLayer = 128u * kRowBytes;
+    constexpr uint32_t kHid = 0u;                           // 5 x 128 rows: the inputs of layers 1 .. 5
+    constexpr uint32_t kEnc = kHid + 5u * kLayer;           // 64 rows: the encoding
+    constexpr uint32_t kOut = kEnc + 64u * kRowBytes;       // 16 rows: output deltas
+    constexpr uint32_t kDrow = kOut + 16u * kRowBytes;      // two buffers of 128 delta rows
+    constexpr uint32_t kFragAt = kDrow + 2u * kLayer;       // two fragment buffers
+    static_assert(kFragAt + 2u * kGradFrag == kGradDensityLds, "LDS map");
+    lds_byte* const enc = grad_lds + kEnc;
+    lds_byte* const frag = grad_lds + kFragAt;
+    const uint32_t lane = threadIdx.x & 63u, g = lane >> 4, s16 = lane & 15u, wv = wave_index(), wr = wv >> 2, wc = wv & 3u;
+    GradLane L;
+    L.template init<kDrow, kFragAt>(lane, wv);
+    const FragSrc S       = frag_src(frags, lane);
+    const uint32_t n      = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
+    const uint32_t groups = (n + 63u) / 64u;
+    floatx4 w0[4][1], w1[4][2], w2[4][2], w3[4][2], w4[4][2], w5 = {0.0f, 0.0f, 0.0f, 0.0f};
+    grad_dw_zero(w0);
+    grad_dw_zero(w1);
+    grad_dw_zero(w2);
+    grad_dw_zero(w3);
+    grad_dw_zero(w4);
+    for (uint32_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+        const uint32_t s0 = gi * 64u;
+        L.hide();
+        half8_t a2[2], a4[4], a1[1];
+        floatx4 acc[4];
+        grad_weights(S, kRefLayers[0].frag0, wv, a2);
+        __syncthreads();  // the previous group's readers are done
+        {
+            float p[3], d[3];
+            grad_point<kFromSamples>(in, min(s0 + lane, n - 1u), p, d);
+            grad_encode<10u>(p, wv, [&](uint32_t k, half_t v) {
+                frag_put_identity(frag, k, lane, v);
+                row_put(enc, k, lane, v);
+            });
+            if (wv == 7u) {
+                frag_put_identity(frag, 63u, lane, (half_t)0.0f);
+                row_put(enc, 63u, lane, (half_t)0.0f);
+            }
+        }
+        // The output deltas' rows: tile wc by waves 0..3.
+        const half4_t* dp = reinterpret_cast<const half4_t*>(deltas + (uint64_t)(s0 + s16) * 16u + 4u * g);  // tile t: + 64 t
+        if (wr == 0u) {
+            const half4_t h = dp[64u * wc];
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) row_put(grad_lds + kOut, 4u * g + e, 16u * wc + s16, h[e]);
+        }
+        __syncthreads();
+        // Each step: the product, the request for the next step's weights
+        // (in flight across the rest of the step), its results.
+        grad_product(a2, 0u, L, acc);
+        grad_weights(S, kRefLayers[1].frag0, wv, a4);
+        const uint32_t m0 = grad_emit<true, true>(acc, L, 1u, kHid);
+        __syncthreads();
+        grad_product(a4, 1u, L, acc);
+        grad_weights(S, kRefLayers[2].frag0, wv, a4);
+        const uint32_t m1 = grad_emit<true, true>(acc, L, 0u, kHid + kLayer);
+        __syncthreads();
+        grad_product(a4, 0u, L, acc);
+        grad_weights(S, kRefLayers[3].frag0, wv, a4);
+        const uint32_t m2 = grad_emit<true, true>(acc, L, 1u, kHid + 2u * kLayer);
+        __syncthreads();
+        grad_product(a4, 1u, L, acc);
+        grad_weights(S, kRefLayers[4].frag0, wv, a4);
+        const uint32_t m3 = grad_emit<true, true>(acc, L, 0u, kHid + 3u * kLayer);
+        grad_weights(S, kRefT[4].frag0, wv, a1);
+        half4_t d5[4];
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) d5[t] = dp[64u * t];
+        __syncthreads();
+        grad_product(a4, 0u, L, acc);
+        grad_weights(S, kRefT[5].frag0, wv, a4);
+        const uint32_t m4 = grad_emit<false, true>(acc, L, 0u, kHid + 4u * kLayer);
+        // delta of layer 4's outputs (needs no other wave's results).
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) acc[t] = mfma16x16x32(a1[0], half8_t{d5[t][0], d5[t][1], d5[t][2], d5[t][3], 0, 0, 0, 0}, floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+        grad_emit_delta<true>(acc, m4, L, 1u, kDrow);
+        __syncthreads();
+        grad_product(a4, 1u, L, acc);
+        grad_weights(S, kRefT[6].frag0, wv, a4);
+        grad_emit_delta<true>(acc, m3, L, 0u, kDrow + kLayer);
+        grad_dw_output(w5, L, kOut, kHid + 4u * kLayer, wv);
+        grad_dw(w4, L.dlt, 0u, L.in, kHid + 3u * kLayer);
+        __syncthreads();
+        grad_product(a4, 0u, L, acc);
+        grad_weights(S, kRefT[7].frag0, wv, a4);
+        grad_emit_delta<true>(acc, m2, L, 1u, kDrow);
+        grad_dw(w3, L.dlt, kLayer, L.in, kHid + 2u * kLayer);
+        __syncthreads();
+        grad_product(a4, 1u, L, acc);
+        grad_weights(S, kRefT[8].frag0, wv, a4);
+        grad_emit_delta<true>(acc, m1, L, 0u, kDrow + kLayer);
+        grad_dw(w2, L.dlt, 0u, L.in, kHid + kLayer);
+        __syncthreads();
+        grad_product(a4, 0u, L, acc);
+        grad_emit_delta<false>(acc, m0, L, 0u, kDrow);
+        grad_dw(w1, L.dlt, kLayer, L.in, kHid);
+        __syncthreads();
+        {
+            const uint32_t op[2] = {L.in[0] - 16u * kRowBytes * wc, L.in[1] - 16u * kRowBytes * wc};  // 16 columns per wave
+            grad_dw(w0, L.dlt, 0u, op, kEnc);
+        }
+    }
+    float* dst = partial + (uint64_t)blockIdx.x * (kRefDensityParams + kRefColorParams);
+    grad_dw_store(w0, dst + kRefLayers[0].w_off, 64u, 4u * wr, wc, lane);
+    grad_dw_store(w1, dst + kRefLayers[1].w_off, 128u, 4u * wr, 2u * wc, lane);
+    grad_dw_store(w2, dst + kRefLayers[2].w_off, 128u, 4u * wr, 2u * wc, lane);
+    grad_dw_store(w3, dst + kRefLayers[3].w_off, 128u, 4u * wr, 2u * wc, lane);
+    grad_dw_store(w4, dst + kRefLayers[4].w_off, 128u, 4u * wr, 2u * wc, lane);
+    grad_dw_out_store(w5, dst + kRefLayers[5].w_off, wv, lane);
 }
 
 // Composite forward + backward with the reference's loss (:1095-1182), one
@@ -983,14 +1465,12 @@ hipError_t ref_pack_weights(const half_t* dparams, const half_t* cparams, half8_
     return hipGetLastError();
 }
 
-hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_t n, float4* out, float4* raw, hipStream_t stream) {
+static uint32_t ref_field_blocks(uint32_t n) { return min(((n + 63u) / 64u + kBlockWaves - 1u) / kBlockWaves, device_cu_count() * 2u); }
+
+hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_t n, float4* out, float4* raw, hipStream_t stream, half_t* dens_out) {
     if (n == 0u) return hipSuccess;
-    const uint32_t groups = (n + 63u) / 64u;
-    const uint32_t need   = (groups + kBlockWaves - 1u) / kBlockWaves;
-    const uint32_t cap    = device_cu_count() * 2u;
-    const uint32_t blocks = need < cap ? need : cap;
-    if (in.samples) k_ref_field<true><<<blocks, kBlockThreads, 0, stream>>>(frags, in, n, out, raw);
-    else k_ref_field<false><<<blocks, kBlockThreads, 0, stream>>>(frags, in, n, out, raw);
+    if (in.samples) k_ref_field<true><<<ref_field_blocks(n), kBlockThreads, 0, stream>>>(frags, in, n, out, raw, dens_out);
+    else k_ref_field<false><<<ref_field_blocks(n), kBlockThreads, 0, stream>>>(frags, in, n, out, raw, dens_out);
     return hipGetLastError();
 }
 
@@ -1004,16 +1484,31 @@ hipError_t launch_ref_composite_train(const RefTrainLaunch& T, const uint32_t* k
     return hipGetLastError();
 }
 
-hipError_t launch_ref_backward_train(const RefTrainLaunch& T, const FieldInputs& in, const float4* draw, float loss_scale, float* grad, double* norm, hipStream_t st) {
-    const uint32_t need = T.np / 64u / kBlockWaves + 1u, cap = device_cu_count() * 2u;
-    k_ref_backward<true><<<need < cap ? need : cap, kBlockThreads, 0, st>>>(T.frags, in, T.np, draw, loss_scale, T.acts, T.dlts, T.np);
-    hipError_t e = hipGetLastError();
+uint32_t ref_grad_blocks(uint32_t np) { return max(1u, min(np / 64u, device_cu_count())); }
+
+namespace {
+
+template <bool kFromSamples>
+hipError_t launch_ref_grad(const half8_t* frags, const FieldInputs& in, uint32_t n, uint32_t np, const half_t* dens, const float4* draw, float loss_scale, half_t* deltas, float* partial, float* ddensity, float* dcolor, double* norm,
+                           hipStream_t st) {
+    hipError_t e = hipFuncSetAttribute((const void*)k_ref_grad_color<kFromSamples>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGradColorLds);
+    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k_ref_grad_density<kFromSamples>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGradDensityLds);
     if (e != hipSuccess) return e;
-    k_ref_dw<<<10u * T.chunks, kBlockThreads, 0, st>>>(T.acts, T.dlts, T.np, kRefDwChunk, T.chunks, T.partial, in.n_dev);
+    const uint32_t blocks = ref_grad_blocks(np);
+    k_ref_grad_color<kFromSamples><<<blocks, kGradThreads, kGradColorLds, st>>>(frags, in, n, dens, draw, loss_scale, deltas, partial);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_ref_dw_reduce<<<kRefReduceBlocks, 256, 0, st>>>(T.partial, T.chunks, grad, grad + kRefDensityParams, norm);
+    k_ref_grad_density<kFromSamples><<<blocks, kGradThreads, kGradDensityLds, st>>>(frags, in, n, deltas, partial);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_ref_dw_reduce<<<kRefReduceBlocks, 256, 0, st>>>(partial, blocks, ddensity, dcolor, norm);
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_ref_backward_train(const RefTrainLaunch& T, const FieldInputs& in, const float4* draw, float loss_scale, float* grad, double* norm, hipStream_t st) {
+    return launch_ref_grad<true>(T.frags, in, T.np, T.np, T.dens, draw, loss_scale, T.deltas, T.partial, grad, grad + kRefDensityParams, norm, st);
 }
 
 }  // namespace nerf_hip
@@ -1050,7 +1545,7 @@ NERF_API NerfStatus nerf_ext_ref_field_forward(const uint16_t* density_params, c
 
 namespace {
 // nerf_ext_ref_backward, with the neuron-major rows in the caller's buffers
-// when acts_out / dlts_out are given (else in temporary ones).
+// when acts_out and dlts_out are given.
 NerfStatus ref_backward(const char* who, const uint16_t* density_params, const uint16_t* color_params, const float* positions, const float* directions, const float* draw, uint32_t n, float loss_scale, float* ddensity,
                         float* dcolor, uint16_t* acts_out, uint16_t* dlts_out, void* stream) {
     if (n == 0u) return NERF_STATUS_OK;
@@ -1058,33 +1553,38 @@ NerfStatus ref_backward(const char* who, const uint16_t* density_params, const u
     NERF_CHECK_ARG(n <= (1u << 20), std::string(who) + ": at most 2^20 samples per call (buffer descriptors address < 4 GiB)");
     hipStream_t st        = (hipStream_t)stream;
     const uint32_t np     = (n + 63u) / 64u * 64u;
+    const bool rows       = acts_out != nullptr;  // with rows: stored, and multiplied from there
     const uint32_t chunk  = kRefDwChunk;
-    const uint32_t chunks = (np + chunk - 1u) / chunk;
+    const uint32_t chunks = rows ? (np + chunk - 1u) / chunk : ref_grad_blocks(np);
     half8_t* frags = nullptr;
-    half_t *acts = (half_t*)acts_out, *dlts = (half_t*)dlts_out;
+    half_t *acts = (half_t*)acts_out, *dlts = (half_t*)dlts_out, *deltas = nullptr;
     float* partial = nullptr;
     NERF_HIP_TRY(hipMallocAsync((void**)&frags, sizeof(half8_t) * 64u * kRefFragments, st));
-    if (!acts_out) NERF_HIP_TRY(hipMallocAsync((void**)&acts, sizeof(half_t) * (uint64_t)kActRows * np, st));
-    if (!dlts_out) NERF_HIP_TRY(hipMallocAsync((void**)&dlts, sizeof(half_t) * (uint64_t)kDltRows * np, st));
+    if (!rows) NERF_HIP_TRY(hipMallocAsync((void**)&deltas, sizeof(half_t) * 32ull * np, st));
     NERF_HIP_TRY(hipMallocAsync((void**)&partial, sizeof(float) * (uint64_t)chunks * (kRefDensityParams + kRefColorParams), st));
     FieldInputs in{};
     in.positions  = positions;
     in.directions = directions;
     hipError_t e  = ref_pack_weights((const half_t*)density_params, (const half_t*)color_params, frags, st);
-    if (e == hipSuccess) {
+    if (e == hipSuccess && !rows) {
+        k_ref_field<false, true><<<ref_field_blocks(n), kBlockThreads, 0, st>>>(frags, in, n, nullptr, nullptr, deltas + 16ull * np);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess && !rows) e = launch_ref_grad<false>(frags, in, n, np, deltas + 16ull * np, (const float4*)draw, loss_scale, deltas, partial, ddensity, dcolor, nullptr, st);
+    if (e == hipSuccess && rows) {
         const uint32_t need = np / 64u / kBlockWaves + 1u, cap = device_cu_count() * 2u;
-        k_ref_backward<false><<<need < cap ? need : cap, kBlockThreads, 0, st>>>(frags, in, n, (const float4*)draw, loss_scale, acts, dlts, np);
+        k_ref_backward<<<need < cap ? need : cap, kBlockThreads, 0, st>>>(frags, in, n, (const float4*)draw, loss_scale, acts, dlts, np);
         e = hipGetLastError();
+        if (e == hipSuccess) {
+            k_ref_dw<<<10u * chunks, kBlockThreads, 0, st>>>(acts, dlts, np, chunk, chunks, partial);
+            e = hipGetLastError();
+        }
+        if (e == hipSuccess) {
+            k_ref_dw_reduce<<<kRefReduceBlocks, 256, 0, st>>>(partial, chunks, ddensity, dcolor, nullptr);
+            e = hipGetLastError();
+        }
     }
-    if (e == hipSuccess) {
-        k_ref_dw<<<10u * chunks, kBlockThreads, 0, st>>>(acts, dlts, np, chunk, chunks, partial, nullptr);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-        k_ref_dw_reduce<<<kRefReduceBlocks, 256, 0, st>>>(partial, chunks, ddensity, dcolor, nullptr);
-        e = hipGetLastError();
-    }
-    const hipError_t f[4] = {hipFreeAsync(partial, st), dlts_out ? hipSuccess : hipFreeAsync(dlts, st), acts_out ? hipSuccess : hipFreeAsync(acts, st), hipFreeAsync(frags, st)};
+    const hipError_t f[3] = {hipFreeAsync(partial, st), deltas ? hipFreeAsync(deltas, st) : hipSuccess, hipFreeAsync(frags, st)};
     NERF_HIP_TRY(e);
     for (hipError_t x : f) NERF_HIP_TRY(x);
     return NERF_STATUS_OK;

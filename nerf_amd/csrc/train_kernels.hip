@@ -2148,7 +2148,7 @@ static hipError_t launch_ref_train_stage(const TrainParams& P, const TrainBuffer
             k_occ_bits<<<(P.occ_cells + 255u) / 256u, 256, 0, st>>>(P, B.state, B.occ_window, B.density, B.bits);
         }
         break;
-    case NERF_EXT_STAGE_FORWARD: return launch_ref_field(B.ref.frags, in, P.sample_cap, B.field, nullptr, st);
+    case NERF_EXT_STAGE_FORWARD: return launch_ref_field(B.ref.frags, in, P.sample_cap, B.field, nullptr, st, B.ref.dens);
     case NERF_EXT_STAGE_COMPOSITE: return launch_ref_composite_train(B.ref, B.kept, B.offsets, B.samples, B.field, B.gt, B.draw, &B.state->loss_sum, &B.state->n_rays, &B.state->n_active, st);
     case NERF_EXT_STAGE_BACKWARD: {
         const hipError_t e = launch_ref_backward_train(B.ref, in, B.draw, P.loss_scale, B.mlp_grad, B.norm_partials, st);

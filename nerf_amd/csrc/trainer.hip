@@ -245,12 +245,11 @@ NerfStatus trainer_create(const NerfExtTrainDesc* d, const BorrowedModel* borrow
     if (ref) {
         RefTrainLaunch& R = B.ref;
         R.np              = (P.sample_cap + 63u) / 64u * 64u;
-        R.chunks          = (R.np + kRefDwChunk - 1u) / kRefDwChunk;
         R.max_rays        = P.max_rays;
         NERF_HIP_TRY(alloc(T, R.frags, 64ull * kRefFragments));
-        NERF_HIP_TRY(alloc(T, R.acts, (uint64_t)kRefActRows * R.np));
-        NERF_HIP_TRY(alloc(T, R.dlts, (uint64_t)kRefDltRows * R.np));
-        NERF_HIP_TRY(alloc(T, R.partial, (uint64_t)R.chunks * kRefParams));
+        NERF_HIP_TRY(alloc(T, R.dens, 16ull * R.np));
+        NERF_HIP_TRY(alloc(T, R.deltas, 16ull * R.np));
+        NERF_HIP_TRY(alloc(T, R.partial, (uint64_t)ref_grad_blocks(R.np) * kRefParams));
         B.occ_window = P.occ_cells_per_update < P.occ_cells ? P.occ_cells_per_update : P.occ_cells;
         NERF_HIP_TRY(alloc(T, B.occ_points, 3ull * B.occ_window));
         NERF_HIP_TRY(alloc(T, B.occ_dirs, 3ull * B.occ_window));
