@@ -1129,41 +1129,52 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(2,
     grad_dw_zero(w6);
     grad_dw_zero(w7);
     grad_dw_zero(w8);
-    for (uint32_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+    // What a group starts from, requested two steps before the previous one
+    // ends: its directions, the density outputs of tile wc (waves 4..7), the
+    // output gradients (lane group 0), the first weights.
+    float p[3], d[3];
+    half4_t ho = {0, 0, 0, 0};
+    float4 dr[4];
+    half8_t a2[2];
+    auto fetch = [&](uint32_t gi) {
         const uint32_t s0 = gi * 64u;
-        L.hide();
-        half8_t a2[2], a4[4], a1[1];
-        floatx4 acc[4];
-        grad_weights(S, kRefLayers[6].frag0, wv, a2);
-        __syncthreads();  // the previous group's readers are done (and the zero fill)
-        {
-            float p[3], d[3];
-            grad_point<kFromSamples>(in, min(s0 + lane, n - 1u), p, d);
-            grad_encode<4u>(d, wv, [&](uint32_t k, half_t v) {
-                frag_put_direction(dfrag, k, lane, v);
-                row_put(cin, 15u + k, lane, v);
-            });
-        }
-        // The output deltas: lane group 0's four of each tile as operands, and
-        // the three used rows.
-        half8_t d9[4];
+        grad_point<kFromSamples>(in, min(s0 + lane, n - 1u), p, d);
+        if (wr == 1u) ho = *reinterpret_cast<const half4_t*>(dens + (uint64_t)min(s0 + 16u * wc + s16, n - 1u) * 16u + 4u * g);
 #pragma unroll
         for (uint32_t t = 0; t < 4u; ++t) {
             const uint32_t st = s0 + 16u * t + s16;
-            const float4 dr   = g == 0u && st < n ? draw[st] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            d9[t]             = half8_t{to_half_rne(loss_scale * dr.y), to_half_rne(loss_scale * dr.z), to_half_rne(loss_scale * dr.w), 0, 0, 0, 0, 0};
+            dr[t]             = g == 0u && st < n ? draw[st] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        grad_weights(S, kRefLayers[6].frag0, wv, a2);
+    };
+    if (blockIdx.x < groups) fetch(blockIdx.x);
+    for (uint32_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+        L.hide();
+        half8_t a4[4], a1[1];
+        floatx4 acc[4];
+        __syncthreads();  // the previous group's readers are done (and the zero fill)
+        grad_encode<4u>(d, wv, [&](uint32_t k, half_t v) {
+            frag_put_direction(dfrag, k, lane, v);
+            row_put(cin, 15u + k, lane, v);
+        });
+        // The output deltas: operands of every tile, and the three used rows.
+        half8_t d9[4];
+        half_t dsig = (half_t)0.0f;  // of tile wc
+#pragma unroll
+        for (uint32_t t = 0; t < 4u; ++t) {
+            d9[t] = half8_t{to_half_rne(loss_scale * dr[t].y), to_half_rne(loss_scale * dr[t].z), to_half_rne(loss_scale * dr[t].w), 0, 0, 0, 0, 0};
+            if (t == wc) dsig = to_half_rne(loss_scale * dr[t].x);
             if (g == 0u && t == wc && wr == 0u) {
 #pragma unroll
                 for (uint32_t e = 0; e < 3u; ++e) row_put(dout, e, 16u * t + s16, d9[t][e]);
             }
         }
-        // Density outputs: tile wc by waves 4..7, into the colour input.
+        // Density outputs into the colour input.
         if (wr == 1u) {
-            const half4_t h = *reinterpret_cast<const half4_t*>(dens + (uint64_t)min(s0 + 16u * wc + s16, n - 1u) * 16u + 4u * g);
-            *reinterpret_cast<half4_t*>(dfrag + 1024u * wc + 16u * lane) = h;
+            *reinterpret_cast<half4_t*>(dfrag + 1024u * wc + 16u * lane) = ho;
 #pragma unroll
             for (uint32_t e = 0; e < 4u; ++e)
-                if (4u * g + e >= 1u) row_put(cin, 4u * g + e - 1u, 16u * wc + s16, h[e]);
+                if (4u * g + e >= 1u) row_put(cin, 4u * g + e - 1u, 16u * wc + s16, ho[e]);
         }
         __syncthreads();
         // Each step: the product, the request for the next step's weights
@@ -1190,6 +1201,7 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(2,
         grad_emit_delta<true>(acc, m7, L, 1u, kDrow + kLayer);
         grad_dw_output(w9, L, kOut, kHid + 2u * kLayer, wv);
         grad_dw(w8, L.dlt, 0u, L.in, kHid + kLayer);
+        fetch(gi + gridDim.x);
         __syncthreads();
         grad_product(a4, 1u, L, acc);
         grad_weights(S, kRefT[3].frag0, 0u, a4);
@@ -1204,10 +1216,9 @@ __global__ __launch_bounds__(kGradThreads) __attribute__((amdgpu_waves_per_eu(2,
             floatx4 o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (uint32_t q = 0; q < 4u; ++q) o = mfma16x16x32(a4[q], frag_read(0u, L, q, wc), o);
-            const uint32_t st = s0 + 16u * wc + s16;
-            half4_t h         = half4_t{to_half_rne(o[0]), to_half_rne(o[1]), to_half_rne(o[2]), to_half_rne(o[3])};
-            if (g == 0u) h[0] = to_half_rne(loss_scale * (st < n ? draw[st].x : 0.0f));
-            *reinterpret_cast<half4_t*>(deltas + (uint64_t)st * 16u + 4u * g) = h;
+            half4_t h = half4_t{to_half_rne(o[0]), to_half_rne(o[1]), to_half_rne(o[2]), to_half_rne(o[3])};
+            if (g == 0u) h[0] = dsig;
+            *reinterpret_cast<half4_t*>(deltas + (uint64_t)(gi * 64u + 16u * wc + s16) * 16u + 4u * g) = h;
         }
     }
     float* dst = partial + (uint64_t)blockIdx.x * (kRefDensityParams + kRefColorParams) + kRefDensityParams;
