@@ -146,3 +146,30 @@ def test_ref_layers_from_gpu_rows(scale, n):
         rel = np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-30)
         print(f"[layer] dW layer {l}: relative Frobenius {rel:.3e}", flush=True)
         assert rel <= 1e-4, f"dW layer {l}: relative Frobenius error {rel:.3e}"
+
+
+# One sample; the edges of a 64-sample group; more groups than workgroups (a
+# workgroup's second group); a ragged last group.
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257 * 64, 300 * 64 + 17])
+def test_ref_gradients_match_stored_rows(n):
+    announce(f"reference-model weight gradients, fused against stored rows, n={n}")
+    m = ext.RefModel.create(ext.ref_mlp_init(0) * 1.5, ext.ref_mlp_init(1) * 1.5)
+    draw = np.random.default_rng(63).normal(0, 1e-2, (n, 4)).astype(np.float32)
+    np_ = (n + 63) // 64 * 64
+    d_p, d_d, d_r = DeviceArray.from_numpy(world_points(n, 61)), DeviceArray.from_numpy(unit_dirs(n, 62)), DeviceArray.from_numpy(draw)
+    acts, dlts = DeviceArray((ACT_ROWS * np_,), np.uint16), DeviceArray((DLT_ROWS * np_,), np.uint16)
+    got, want = [[DeviceArray((k,), np.float32) for k in (75776, 40960)] for _ in range(2)]
+    L.call("nerf_ext_ref_backward_rows", m.density.ptr, m.color.ptr, d_p.ptr, d_d.ptr, d_r.ptr, n, LOSS_SCALE, want[0].ptr, want[1].ptr, acts.ptr, dlts.ptr, None)
+    L.call("nerf_ext_ref_backward", m.density.ptr, m.color.ptr, d_p.ptr, d_d.ptr, d_r.ptr, n, LOSS_SCALE, got[0].ptr, got[1].ptr, None)
+    synchronize()
+    A, D = _rows(acts.numpy(), ACT_ROWS, n), _rows(dlts.numpy(), DLT_ROWS, n)
+    gamma = n * 2.0 ** -24  # Higham's bound on each fp32 sum of n products (exact fp16 x fp16)
+    for net, layers in ((0, range(6)), (1, range(6, 10))):
+        g, w, off = got[net].numpy().astype(np.float64), want[net].numpy().astype(np.float64), 0
+        for l in layers:
+            o, i = SHAPES[l]
+            S = np.abs(D[DLT_OFF[l]:DLT_OFF[l] + o]) @ np.abs(A[ACT_OFF[l]:ACT_OFF[l] + i]).T
+            diff = np.abs(g[off:off + o * i] - w[off:off + o * i]).reshape(o, i)
+            assert np.all(diff <= 2.0 * gamma * S + 1e-30), f"layer {l}: {np.max(diff - 2.0 * gamma * S)}"
+            off += o * i
+        assert off == g.size and np.any(g != 0.0)
