@@ -579,6 +579,8 @@ struct FieldWeights {
 // Level-split encode of a march sample stream: features [cap][32] fp16 rows,
 // or with lm, level-major fp16 pairs lm[level * cap + sample].
 hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const FieldInputs& in, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream);
+// The same for an array of points in the unit cube, level-major.
+hipError_t launch_encode_positions(const GridParams& g, const half_t* table, const float* positions, uint32_t n, uint32_t* lm, hipStream_t stream);
 // Fills the cell tables of levels [0, t.levels) from the hash table (fp16).
 hipError_t build_cell_tables(const GridParams& g, const half_t* table, const CellTables& t, hipStream_t stream);
 // out4 [n] float4 (sigma, r, g, b).
@@ -624,5 +626,16 @@ hipError_t launch_ref_backward_train(const RefTrainLaunch& T, const FieldInputs&
 
 // Number of compute units of the current device (cached).
 uint32_t device_cu_count();
+
+// Temporary device memory of one call, in stream order, from a memory pool of
+// the library's (one per GPU): a released block stays in the pool for the
+// next call up to kScratchKept bytes per GPU, where the default pool gives it
+// back to the system at the next synchronisation and the call after that
+// allocates anew.  scratch_trim gives the current GPU's unused blocks back;
+// the destroy calls of the library's objects do, and an allocation that fails
+// does before it is tried once more.  Safe from any thread, for any stream.
+constexpr uint64_t kScratchKept = 192ull << 20;
+hipError_t scratch_alloc(void** p, uint64_t bytes, hipStream_t stream);
+void scratch_trim();
 
 }  // namespace nerf_hip

@@ -1540,7 +1540,7 @@ NERF_API NerfStatus nerf_ext_ref_field_forward(const uint16_t* density_params, c
     NERF_CHECK_ARG(density_params && color_params && positions && directions && out, "nerf_ext_ref_field_forward: null pointer");
     hipStream_t st  = (hipStream_t)stream;
     half8_t* frags = nullptr;
-    NERF_HIP_TRY(hipMallocAsync((void**)&frags, sizeof(half8_t) * 64u * kRefFragments, st));
+    NERF_HIP_TRY(scratch_alloc((void**)&frags, sizeof(half8_t) * 64u * kRefFragments, st));
     FieldInputs in{};
     in.positions  = positions;
     in.directions = directions;
@@ -1570,9 +1570,9 @@ NerfStatus ref_backward(const char* who, const uint16_t* density_params, const u
     half8_t* frags = nullptr;
     half_t *acts = (half_t*)acts_out, *dlts = (half_t*)dlts_out, *deltas = nullptr;
     float* partial = nullptr;
-    NERF_HIP_TRY(hipMallocAsync((void**)&frags, sizeof(half8_t) * 64u * kRefFragments, st));
-    if (!rows) NERF_HIP_TRY(hipMallocAsync((void**)&deltas, sizeof(half_t) * 32ull * np, st));
-    NERF_HIP_TRY(hipMallocAsync((void**)&partial, sizeof(float) * (uint64_t)chunks * (kRefDensityParams + kRefColorParams), st));
+    NERF_HIP_TRY(scratch_alloc((void**)&frags, sizeof(half8_t) * 64u * kRefFragments, st));
+    if (!rows) NERF_HIP_TRY(scratch_alloc((void**)&deltas, sizeof(half_t) * 32ull * np, st));
+    NERF_HIP_TRY(scratch_alloc((void**)&partial, sizeof(float) * (uint64_t)chunks * (kRefDensityParams + kRefColorParams), st));
     FieldInputs in{};
     in.positions  = positions;
     in.directions = directions;

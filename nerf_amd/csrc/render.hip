@@ -830,6 +830,7 @@ NERF_API NerfStatus nerf_ext_renderer_destroy(NerfExtRenderer* renderer) {
     if (!renderer) return NERF_STATUS_OK;
     (void)hipDeviceSynchronize();
     delete renderer;
+    scratch_trim();
     return NERF_STATUS_OK;
 }
 

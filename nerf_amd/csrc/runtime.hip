@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <mutex>
+
 #include "common.hpp"
 
 namespace nerf_hip {
@@ -31,6 +33,60 @@ uint32_t device_cu_count() {
         cached_device = dev;
     }
     return cached;
+}
+
+namespace {
+
+constexpr int kScratchDevices = 64;
+std::mutex g_scratch_mutex;
+hipMemPool_t g_scratch_pool[kScratchDevices];
+
+// The current GPU's pool (created by the first call there unless !create), or null.
+hipError_t scratch_pool(bool create, hipMemPool_t* out) {
+    int dev      = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kScratchDevices) return hipErrorInvalidDevice;
+    std::scoped_lock lock(g_scratch_mutex);
+    if (!g_scratch_pool[dev] && create) {
+        hipMemPoolProps props{};
+        props.allocType     = hipMemAllocationTypePinned;
+        props.handleTypes   = hipMemHandleTypeNone;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id   = dev;
+        hipMemPool_t pool   = nullptr;
+        e                   = hipMemPoolCreate(&pool, &props);
+        if (e != hipSuccess) return e;
+        uint64_t kept = kScratchKept;
+        e             = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &kept);
+        if (e != hipSuccess) {
+            (void)hipMemPoolDestroy(pool);
+            return e;
+        }
+        g_scratch_pool[dev] = pool;
+    }
+    *out = g_scratch_pool[dev];
+    return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t scratch_alloc(void** p, uint64_t bytes, hipStream_t stream) {
+    hipMemPool_t pool = nullptr;
+    hipError_t e      = scratch_pool(true, &pool);
+    if (e != hipSuccess) return e;
+    e = hipMallocFromPoolAsync(p, bytes, pool, stream);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        (void)hipMemPoolTrimTo(pool, 0);
+        e = hipMallocFromPoolAsync(p, bytes, pool, stream);
+    }
+    return e;
+}
+
+void scratch_trim() {
+    hipMemPool_t pool = nullptr;
+    if (scratch_pool(false, &pool) == hipSuccess && pool) (void)hipMemPoolTrimTo(pool, 0);
 }
 
 }  // namespace nerf_hip

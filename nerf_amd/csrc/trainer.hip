@@ -428,6 +428,7 @@ NERF_API NerfStatus nerf_ext_trainer_destroy(NerfExtTrainer* trainer) {
     if (!trainer) return NERF_STATUS_OK;
     delete trainer->t;
     delete trainer;
+    scratch_trim();
     return NERF_STATUS_OK;
 }
 
