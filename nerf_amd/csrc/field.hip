@@ -502,6 +502,30 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
             k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromRows{in.features_out}, dirs, out4);
         return hipGetLastError();
     }
+    // Points from an array, which may lie anywhere (a wave's gathers then share
+    // no lines, and all levels together do not fit an XCD's L2): encoded level
+    // group by level group, then the MLPs over the features, when that is
+    // faster.  Random points, fused against split: T = 2^19: 2^14 points 17.6
+    // / 20.6 us, 2^16 53 / 31, 300,007 222 / 109, 2^20 710 / 350; T = 2^17:
+    // 2^16 36 / 30, 2^20 377 / 306; T = 2^15: 2^16 30 / 28, 2^20 269 / 279.
+    // (Points in march order measure the same either way up to 2^20, and much
+    // faster in the level-major kernel beyond, 0.1 against 0.35 ns each, which
+    // therefore keeps the larger arrays.)  The fused kernel needs no memory: a
+    // stream under capture and a failed allocation take it.
+    if (!from_samples && !in.n_dev && !in.features_out && g.table_dtype == NERF_EXT_F16 && g.n_levels == 16u && n <= (1u << 20) && n >= (g.table_size > (1u << 17) ? 1u << 15 : 1u << 16) && g.table_size >= (1u << 17)) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        uint32_t* lm                   = nullptr;
+        if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone && scratch_alloc((void**)&lm, 64ull * n, stream) == hipSuccess) {
+            hipError_t e = launch_encode_positions(g, (const half_t*)table, in.positions, n, lm, stream);
+            if (e == hipSuccess) {
+                k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromLevels{lm, n}, DirsFromArray{in.directions, n}, out4);
+                e = hipGetLastError();
+            }
+            const hipError_t f = hipFreeAsync(lm, stream);
+            return e != hipSuccess ? e : f;
+        }
+        (void)hipGetLastError();
+    }
 #define NERF_FIELD_LAUNCH(K)                                                                                                                   \
     do {                                                                                                                                       \
         if (g.table_dtype == NERF_EXT_F32) {                                                                                                   \

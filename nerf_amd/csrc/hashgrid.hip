@@ -247,10 +247,12 @@ hipError_t build_cell_tables(const GridParams& g, const half_t* table, const Cel
     return hipGetLastError();
 }
 
-hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const FieldInputs& in, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream) {
+namespace {
+
+template <typename Points>
+hipError_t launch_encode_split(const GridParams& g, const half_t* table, const Points& src, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream) {
     if (cap == 0u) return hipSuccess;
     if (g.n_levels != 16u || g.table_dtype != NERF_EXT_F16) return hipErrorInvalidValue;
-    PointsFromSamples src{in.samples, in.sample_ray, in.rays, in.n_dev, cap, {in.bmin[0], in.bmin[1], in.bmin[2]}, {in.bmax[0], in.bmax[1], in.bmax[2]}};
     const uint64_t level_bytes = (uint64_t)g.table_size * g.n_features * 2u;
     const uint32_t blocks_256  = (cap + 255u) / 256u;
     // Four levels per XCD when four fit in half of its L2; else one level per
@@ -259,13 +261,26 @@ hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const
     // with T = 2^19 fp16 a level is 2 MiB, and two of them (4 MiB) left no
     // room in the XCD's L2 for the feature rows streaming through it (the
     // reference host's 4,096 rays x <= 64 steps: 117 us for two levels per
-    // XCD, 95 us for the two phases as two launches).
+    // XCD, 95 us for the two phases as two launches).  Levels dealt to the
+    // XCDs in eighths of their total cost, so that all finish together,
+    // measured no faster: an XCD then reads parts of three levels (300,007
+    // random points with the MLP pass: 125 us against 109).
     if (4u * level_bytes <= (2ull << 20)) {
         k_encode_split<half_t, half_t, 4u><<<8u * ((blocks_256 + 1u) / 2u), 256, 0, stream>>>(g, table, src, features, false, 0u, lm, cap);
     } else {
         k_encode_split<half_t, half_t, 1u><<<16u * blocks_256, 256, 0, stream>>>(g, table, src, features, false, 2u, lm, cap);
     }
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const FieldInputs& in, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream) {
+    return launch_encode_split(g, table, PointsFromSamples{in.samples, in.sample_ray, in.rays, in.n_dev, cap, {in.bmin[0], in.bmin[1], in.bmin[2]}, {in.bmax[0], in.bmax[1], in.bmax[2]}}, cap, features, lm, stream);
+}
+
+hipError_t launch_encode_positions(const GridParams& g, const half_t* table, const float* positions, uint32_t n, uint32_t* lm, hipStream_t stream) {
+    return launch_encode_split(g, table, PointsFromArray{positions, n}, n, nullptr, lm, stream);
 }
 
 }  // namespace nerf_hip

@@ -159,3 +159,23 @@ def test_split_encode_then_mlp_equals_fused_field(log2_t):
     synchronize()
     diff = np.count_nonzero(split.numpy().view(np.uint32) != fused.numpy().view(np.uint32))
     assert diff == 0, f"{diff} of {4 * n} values differ"
+
+
+# Point arrays of 2^15 (2^16 at T = 2^17) to 2^20 points take the level-split
+# encode and the MLP pass, smaller ones and captured streams the fused kernel:
+# both sides of each limit, ragged counts, one and four levels per XCD.
+@pytest.mark.parametrize("log2_t,n", [(17, 1 << 16), (17, (1 << 16) + 77), (18, 1 << 15), (19, (1 << 15) + 1), (20, 40007), (19, 1 << 20)])
+def test_field_forward_split_equals_fused(log2_t, n):
+    announce(f"field forward by level split against the fused kernel, T=2^{log2_t}, n={n}")
+    desc = ext.grid_desc(log2_t, L.NERF_EXT_F16)
+    model = ext.Model.create(desc, seed=6, table_range=1.0)
+    pos, dirs = points(n, seed=31), unit_dirs(n, seed=32)
+    d_pos, d_dir, d_o, d_f = DeviceArray.from_numpy(pos), DeviceArray.from_numpy(dirs), DeviceArray((n, 4), np.float32), DeviceArray((n, 4), np.float32)
+    ms = model.struct()
+    L.call("nerf_ext_field_forward", byref(ms), d_pos.ptr, d_dir.ptr, n, d_o.ptr, None)
+    piece = 12000  # below the limit: the fused kernel
+    for a in range(0, n, piece):
+        L.call("nerf_ext_field_forward", byref(ms), d_pos.ptr + 12 * a, d_dir.ptr + 12 * a, min(piece, n - a), d_f.ptr + 16 * a, None)
+    synchronize()
+    diff = np.count_nonzero(d_o.numpy().view(np.uint32) != d_f.numpy().view(np.uint32))
+    assert diff == 0, f"{diff} of {4 * n} values differ"
