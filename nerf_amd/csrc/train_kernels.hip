@@ -1201,8 +1201,7 @@ __device__ __forceinline__ half8_t op_frag(const half_t* ops, uint32_t row0, uin
 // features: rows [n][32], or (features_lm non-null) level-major pairs
 // [16][sample_cap].
 __global__ __launch_bounds__(kThreads) void k_bwd_dx(TrainParams P, const TrainDevState* S, const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, const half_t* __restrict__ features,
-                                                     const uint32_t* __restrict__ features_lm, const float4* __restrict__ draw,
-                                                     const float2* __restrict__ samples, const uint32_t* __restrict__ sample_ray, const float4* __restrict__ rays, float2* __restrict__ dfeat, float* __restrict__ partials) {
+                                                     const uint32_t* __restrict__ features_lm, const float4* __restrict__ draw, const uint32_t* __restrict__ sample_ray, const float4* __restrict__ rays, float2* __restrict__ dfeat, float* __restrict__ partials) {
     extern __shared__ __align__(16) half_t dyn[];
     half8_t* F  = reinterpret_cast<half8_t*>(dyn);
     half_t* ops = dyn + kDxFragBytes / 2u;
@@ -1224,26 +1223,45 @@ __global__ __launch_bounds__(kThreads) void k_bwd_dx(TrainParams P, const TrainD
     // barriers); a wave past the last tile runs one with zero deltas.
     const uint32_t first = blockIdx.x * kWaves, stride = gridDim.x * kWaves;
     const uint32_t iters = tiles > first ? (tiles - first + stride - 1u) / stride : 0u;
-    for (uint32_t it = 0; it < iters; ++it) {
+    // A tile's inputs (the ray's direction, the features, the output
+    // gradients) are requested while the previous tile's weight-gradient
+    // phases run, instead of behind the sample -> ray -> direction chain at the
+    // top of every iteration (2^18 samples: 48.4 -> 46.9 us).
+    struct TileIn {
+        float d[3];
+        half8_t x;
+        float4 gr;
+    };
+    auto fetch = [&](uint32_t it, TileIn& in) {
         const uint32_t tile = first + wave + it * stride;
         const uint32_t s    = tile * 16u + s16;
         const bool live     = tile < tiles && s < n;
         const uint32_t q    = live ? s : n - 1u;  // n > 0 here
-        float p[3], d[3];
-        sample_geometry(samples, sample_ray, rays, P.bmin, P.bmax, q, p, d);
-        half8_t x;
+        const float4 rd     = rays[2ull * sample_ray[q] + 1ull];
+        in.d[0] = rd.x;
+        in.d[1] = rd.y;
+        in.d[2] = rd.z;
         if (features_lm) {
             uint32_t v[4];
 #pragma unroll
             for (uint32_t j = 0; j < 4u; ++j) v[j] = features_lm[(uint64_t)(4u * grp + j) * P.sample_cap + q];
-            x = __builtin_bit_cast(half8_t, v);
+            in.x = __builtin_bit_cast(half8_t, v);
         } else {
-            x = *reinterpret_cast<const half8_t*>(features + (uint64_t)q * 32u + 8u * grp);
+            in.x = *reinterpret_cast<const half8_t*>(features + (uint64_t)q * 32u + 8u * grp);
         }
-        float4 gr       = draw[q];
-        if (!live) gr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // padding samples add nothing to the weight gradients
+        in.gr = draw[q];
+        if (!live) in.gr = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // padding samples add nothing to the weight gradients
+    };
+    TileIn next{};
+    if (iters > 0u) fetch(0u, next);
+    for (uint32_t it = 0; it < iters; ++it) {
+        const uint32_t tile = first + wave + it * stride;
+        const uint32_t s    = tile * 16u + s16;
+        const bool live     = tile < tiles && s < n;
+        const TileIn in     = next;
         TileGrad T;
-        tile_backward(F, x, d, gr, P.loss_scale, grp, T);
+        tile_backward(F, in.x, in.d, in.gr, P.loss_scale, grp, T);
+        if (it + 1u < iters) fetch(it + 1u, next);
         if (live) {
 #pragma unroll
             for (uint32_t b = 0; b < 2u; ++b) {
@@ -2027,7 +2045,7 @@ hipError_t launch_mlp_backward(const TrainParams& P, const TrainBuffers& B, hipS
         lds_set = true;
     }
     const uint32_t dx_blocks = min(cus * 2u, kDxMaxBlocks);  // two per CU (LDS)
-    k_bwd_dx<<<dx_blocks, kThreads, kDxLds, st>>>(P, B.state, B.dparams, B.cparams, B.features, sparse_features(P, B) ? B.features_lm : nullptr, B.draw, B.samples, B.sample_ray, B.rays, B.dfeat, B.dw_partials);
+    k_bwd_dx<<<dx_blocks, kThreads, kDxLds, st>>>(P, B.state, B.dparams, B.cparams, B.features, sparse_features(P, B) ? B.features_lm : nullptr, B.draw, B.sample_ray, B.rays, B.dfeat, B.dw_partials);
     // Coarse levels: LDS slabs per chunk of samples, summed over the chunks
     // by the gradient reduction; hashed levels: binned.  One launch when both
     // are present.
