@@ -58,18 +58,37 @@ constexpr uint32_t kFieldFrags   = 20u;  // density w1[4] w2[2], colour w1[4] w2
 constexpr uint32_t kMlpWaves     = 4u;   // waves per SIMD the register budget is built for
 
 // Fragment f of the two MLPs for lane `lane`, read from the global parameters
-// element by element (any alignment); same values as load_density /
-// load_color give from the staged copy.
-__device__ half8_t mlp_fragment(const half_t* __restrict__ dp, const half_t* __restrict__ cp, uint32_t f, uint32_t lane) {
-    const uint32_t i = lane & 15u;
-    if (f < 4u) return load_a(dp, 32u, f, 0u, KMap::Identity, lane);
-    if (f < 6u) return load_a(dp + 2048, 64u, 0u, f - 4u, KMap::Hidden, lane);
-    if (f < 10u) return load_a(cp, 32u, f - 6u, 0u, KMap::ColorIn, lane);
-    if (f < 18u) return load_a(cp + 2048, 64u, (f - 10u) >> 1, (f - 10u) & 1u, KMap::Hidden, lane);
+// (any alignment) in the runs of four or eight weights that the k-maps keep
+// together; same values as load_density / load_color give from the staged
+// copy.  As element reads the compiler merged them or not with unrelated
+// changes (2^22 samples of the MLP pass: 104.6 us unmerged, 100.9 merged, 99.9
+// as written here).
+__device__ __forceinline__ half4_t weights4(const half_t* p) {
+    half4_t v;
+    __builtin_memcpy(&v, p, 8);
+    return v;
+}
+__device__ __forceinline__ half8_t weights8(const half_t* lo, const half_t* hi) { return cat(weights4(lo), weights4(hi)); }
+
+__device__ __forceinline__ half8_t mlp_fragment(const half_t* __restrict__ dp, const half_t* __restrict__ cp, uint32_t f, uint32_t lane) {
+    const uint32_t i = lane & 15u, g = lane >> 4;
+    auto hidden = [&](const half_t* row) { return weights8(row + 4u * g, row + 16u + 4u * g); };
+    if (f < 4u) {
+        const half_t* row = dp + (16u * f + i) * 32u + 8u * g;
+        return weights8(row, row + 4u);
+    }
+    if (f < 6u) return hidden(dp + 2048 + i * 64u + 32u * (f - 4u));
+    if (f < 10u) {  // density outputs 4g - 1 .. (lane group 0: a zero, then 0 .. 2), SH coefficients 4g ..
+        const half_t* row = cp + (16u * (f - 6u) + i) * 32u;
+        half4_t o         = weights4(g == 0u ? row : row + 4u * g - 1u);
+        if (g == 0u) o = half4_t{(half_t)0.0f, o[0], o[1], o[2]};
+        return cat(o, weights4(row + 15u + 4u * g));
+    }
+    if (f < 18u) return hidden(cp + 2048 + (16u * ((f - 10u) >> 1) + i) * 64u + 32u * ((f - 10u) & 1u));
     // Colour output: row 4c (c = 1..3) of the MFMA computes colour c - 1,
     // every other row is zero (see load_color).
     const bool used = (i & 3u) == 0u && i != 0u;
-    const half8_t v = load_a(cp + 2048 + 4096 + (used ? (i / 4u - 1u) : 0u) * 64u, 64u, 0u, f - 18u, KMap::Hidden, lane & 48u);
+    const half8_t v = hidden(cp + 2048 + 4096 + (used ? (i / 4u - 1u) : 0u) * 64u + 32u * (f - 18u));
     const half8_t z = {};
     return used ? v : z;
 }
@@ -477,17 +496,20 @@ uint32_t persistent_blocks(uint32_t n, uint32_t per_cu) {
 
 hipError_t launch_field(const GridParams& g, const void* table, const FieldWeights& w, const FieldInputs& in, uint32_t n, float4* out4, hipStream_t stream) {
     if (n == 0u) return hipSuccess;
-    // Renders (more than 2^20 samples) take the level-major kernel, 3
-    // workgroups per CU (its LDS and register budget); training-sized
-    // batches the tile kernel, whose 16-sample tiles leave a shorter tail
-    // when a launch is only one or two rounds of work (2^18 samples: 67 vs
-    // 93 us).  The tile kernel runs 4 workgroups per CU: 2^18 samples are
-    // 16,384 tiles, exactly 4 per wave (67 us; 3 per CU leave 5 or 6 tiles
+    // Renders and other large launches take the level-major kernel, 3
+    // workgroups per CU (its LDS and register budget); small ones the tile
+    // kernel, whose 16-sample tiles leave a shorter tail when a launch is only
+    // a few rounds of work (2^18 training samples: 67 vs 93 us).  A render
+    // round's n is its capacity, of which it fills about a third: 100x75
+    // pixels at 256 steps (1.9 M entries) 274 us per render with tiles, 284
+    // level-major; 160x120 at 512 (9.8 M) 865 / 882; 200x150 at 512 (15.4 M)
+    // 1,458 / 1,441.  The tile kernel runs 4 workgroups per CU: 2^18 samples
+    // are 16,384 tiles, exactly 4 per wave (67 us; 3 per CU leave 5 or 6 tiles
     // per wave, 71 us; 5 and 6 per CU, 77 us).  The level-major kernel
-    // measured no faster with its fragments in LDS (49.9 vs 49.8 ms per
-    // render) and slower with 8-wave workgroups at 4 waves per SIMD (52.5
-    // ms: more waves than its L1 serves).
-    const bool level_major  = n > (1u << 20);
+    // measured slower with 8-wave workgroups at 4 waves per SIMD (52.5 vs
+    // 49.8 ms per 800x800 render: more waves than its L1 serves) and with 4
+    // workgroups per CU (100x75: 295 vs 284 us).
+    const bool level_major  = n > (in.sample_index ? 3u << 22 : 1u << 20);
     const uint32_t blocks   = (persistent_blocks(n, level_major ? 3u : 4u) + 7u) / 8u * 8u;  // whole XCD rounds
     const bool from_samples = in.samples != nullptr;
     if (in.sparse && from_samples && in.features_out && !in.sample_index && !in.alpha_in_order && g.table_dtype != NERF_EXT_F32 && g.n_levels == 16u) {

@@ -1079,6 +1079,7 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
             k_round_composite<<<ray_waves, 256, 0, st>>>(l_cur, n_cur, R->counts.ptr, R->prog.ptr, R->cnt.ptr, R->off.ptr, R->field.ptr, d->min_transmittance, bg, R->state.ptr, rgba8, rgb_f32, R->keep.ptr, Es[nxt],
                                                          r + 2u < n_rounds ? 1u : 0u, d->composited, d->shaded);
             NERF_LAUNCH_CHECK("k_round_composite");
+            if (r + 1u == n_rounds) break;  // no ray is left after the last round
             NERF_HIP_TRY(exclusive_scan_u32(R->keep.ptr, R->koff.ptr, nr, R->scan_tmp.ptr, R->keep_total.ptr, st));
             k_round_compact<<<cblocks, 256, 0, st>>>(l_cur, n_cur, R->keep.ptr, R->koff.ptr, R->keep_total.ptr, l_nxt, n_nxt);
             NERF_LAUNCH_CHECK("k_round_compact");
