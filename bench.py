@@ -62,12 +62,12 @@ FIELD_FLOPS_PER_SAMPLE = 2 * (32 * 64 + 64 * 16) + 2 * (31 * 64 + 64 * 64 + 64 *
 # Traffic beyond L2 of the field kernel per sample on this workload, from
 # rocprofv3 FETCH_SIZE (x 2.0) + WRITE_SIZE (x 1.0) on one 800x800 render, the
 # factors being what the same counters read on a plain conversion kernel of
-# known size (profiles/field_forward_800x800_counters.md): 217.52 GB + 7.83 GB
+# known size (profiles/field_forward_800x800_counters.md): 184.53 GB + 7.83 GB
 # over 486,308,861 samples, summed over the render's dispatches.  The render
 # rounds list samples in spatial order, so neighbouring lanes share the coarse
-# levels' table lines and the traffic stays near the 540 algorithmic bytes
-# (58 % L2 hit).
-FIELD_TRAFFIC_BYTES_PER_SAMPLE = 463
+# levels' cells and the traffic stays below the 540 algorithmic bytes (60 % L2
+# hit).
+FIELD_TRAFFIC_BYTES_PER_SAMPLE = 396
 # Reference-model network per sample, on the reference's own padded shapes
 # (backend-cuda.cu:23-54): density 64x128 + 4 x 128x128 + 128x16, colour
 # 48x128 + 2 x 128x128 + 128x16, two flops per multiply-add.
@@ -167,7 +167,7 @@ def kernel_rooflines(reps_small: int = 200):
     gD, gC = DeviceArray((L.NERF_EXT_REF_DENSITY_PARAMS,), np.float32), DeviceArray((L.NERF_EXT_REF_COLOR_PARAMS,), np.float32)
     ms_b = timed(lambda: L.call("nerf_ext_ref_backward", rm.density.ptr, rm.color.ptr, pos.ptr, dirs.ptr, draw.ptr, nb, 128.0, gD.ptr, gC.ptr, st.handle), 20)
     tfs_b = nb * REF_BACKWARD_FLOPS_PER_SAMPLE / (ms_b / 1e3) / 1e12
-    out["ref_backward_2p18"] = {"kernel": "k_ref_backward + k_ref_dw + k_ref_dw_reduce (reference-model MLP backward: recompute, deltas, weight gradients)", "samples": nb, "ms": round(ms_b, 4), "bound": "mfma",
+    out["ref_backward_2p18"] = {"kernel": "k_ref_field (density) + k_ref_grad_color + k_ref_grad_density + k_ref_dw_reduce (reference-model MLP backward: recompute, deltas, weight gradients)", "samples": nb, "ms": round(ms_b, 4), "bound": "mfma",
                                 "achieved": round(tfs_b, 1), "peak": MFMA_FP16_PEAK_TFS, "unit": "TFLOP/s", "frac": round(tfs_b / MFMA_FP16_PEAK_TFS, 4), "flops_per_sample": REF_BACKWARD_FLOPS_PER_SAMPLE}
     out["ref_field_2p22"] = {"kernel": "k_ref_field (reference-model mode: frequency encoding, density 64-128x5-16, colour 48-128x3-16, fp16 MFMA)", "samples": n, "ms": round(ms, 4), "bound": "mfma", "achieved": round(tfs, 1),
                              "peak": MFMA_FP16_PEAK_TFS, "unit": "TFLOP/s", "frac": round(tfs / MFMA_FP16_PEAK_TFS, 4), "flops_per_sample": REF_FLOPS_PER_SAMPLE}

@@ -855,9 +855,11 @@ __global__ __launch_bounds__(256) void k_ref_dw_reduce(const float* __restrict__
 // forward, back-propagate and multiply the weight gradients from LDS, and
 // keep the network's whole gradient in registers until their last group.
 // Storing every layer's rows for a separate product (k_ref_backward and
-// k_ref_dw, 4.4 KB written and read per sample) was bound by that traffic:
-// 640 us per 2^18 samples; the second forward of the density network costs a
-// fifth more matrix work instead.
+// k_ref_dw, 4.4 KB written and read per sample) is bound by that traffic: 640
+// us per 2^18 samples, against 108 (colour) + 200 (density) + 17 us (reduction)
+// and, where no forward left the density outputs, 38 us for them.  What bounds
+// these: the operand reads from LDS (128 KiB per 128 x 128 product, 1,024
+// cycles where the matrix cores need 512) and the barrier per layer.
 //
 //   k_ref_grad_color    colour forward (from the density outputs that
 //                       k_ref_field left) and backward; writes the density
