@@ -162,8 +162,8 @@ def test_split_encode_then_mlp_equals_fused_field(log2_t):
 
 
 # Point arrays of 2^15 (2^16 at T = 2^17) to 2^20 points take the level-split
-# encode and the MLP pass, smaller ones and captured streams the fused kernel:
-# both sides of each limit, ragged counts, one and four levels per XCD.
+# encode and the MLP pass, smaller ones the fused kernel: both limits, ragged
+# counts, one and four levels per XCD.
 @pytest.mark.parametrize("log2_t,n", [(17, 1 << 16), (17, (1 << 16) + 77), (18, 1 << 15), (19, (1 << 15) + 1), (20, 40007), (19, 1 << 20)])
 def test_field_forward_split_equals_fused(log2_t, n):
     announce(f"field forward by level split against the fused kernel, T=2^{log2_t}, n={n}")
