@@ -115,11 +115,12 @@ __device__ __forceinline__ float corner_weight(const LevelCell& c, uint32_t corn
 }
 
 // Weighted sum of a cell's 8 corner entries (fp16 pairs, corner order).
-// kFma: each product is added in one rounding (v_fma_mix_f32, which reads the
-// fp16 operand directly) instead of a conversion, a product and a sum, 16
-// instructions for 48: the march-sample kernels.  The others keep the
-// two-rounding sums of the oracle, which the encode outputs are compared with
-// bit for bit.
+// kFma, renders only: each product is added in one rounding (v_fma_mix_f32,
+// which reads the fp16 operand directly) instead of a conversion, a product
+// and a sum, 16 instructions for 48 (3 x 1280x720 over five cascades 327 ms
+// with them, 351 ms with rounded products).  Point queries and training steps
+// keep the two-rounding sums of the oracle: they encode a point to the same
+// bits, those of nerf_ext_encode_forward.
 template <bool kFma>
 __device__ __forceinline__ void corner_sum(const LevelCell& c, const uint32_t v[8], float& a0, float& a1) {
     a0 = 0.0f;
@@ -522,6 +523,8 @@ struct FieldInputs {
     // level-split encode writes (each XCD whole lines of its levels) instead
     // of features_out, and the MLP pass reads.
     uint32_t* features_lm;
+    // Renders: corner sums in one rounding per corner (corner_sum's kFma).
+    bool fused_sums;
     // Optional (fp16 table): the leading levels cell by cell (level-major
     // kernel).
     CellTables cells;

@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_density_forward(GridParams g,
 // batch (2^18 samples, one ray's consecutive samples per tile) the gathers
 // of a tile then get more registers in flight, 75 -> 71 us at the same 3
 // workgroups per CU.
-template <typename TableT, bool kFromSamples>
+template <typename TableT, bool kFromSamples, bool kFma>
 __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, const TableT* __restrict__ table, const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, FieldInputs in, uint32_t n_cap, float4* __restrict__ out) {
     const uint32_t n = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
     __shared__ __align__(16) half8_t frag[kFieldFrags][kWaveSize];
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, c
             }
         }
         float feat[8];
-        encode_quad<TableT, kFromSamples>(g, table, p, grp, feat);
+        encode_quad<TableT, kFma>(g, table, p, grp, feat);
         const half8_t x = to_half8(feat);
         if (in.features_out && s < n) *reinterpret_cast<half8_t*>(in.features_out + (uint64_t)s * 32u + 8u * grp) = x;
         floatx4 o, c;
@@ -233,15 +233,15 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, c
 // The levels run in rolled loops of two (16 unrolled bodies with three paths
 // each held so many uniform values that 190 of them went through spill lanes,
 // 2,700 vector instructions per group of 64 samples against 2,100), the
-// corner sums take v_fma_mix_f32 (corner_sum), and an incoherent level's
-// entries are fetched as aligned pairs (entry_pair).  Together, 800x800
-// render 44.4 -> 40.9 ms, three 1280x720 views over five cascades
+// corner sums of renders take v_fma_mix_f32 (corner_sum), and an incoherent
+// level's entries are fetched as aligned pairs (entry_pair).  Together,
+// 800x800 render 44.4 -> 40.9 ms, three 1280x720 views over five cascades
 // 471 -> 373 ms.
 // The fp16 features go through LDS (rows of 80 bytes, 16-byte reads of lane
 // group g's levels 4g..4g+3) into the MLP's B-operand layout, four 16-sample
 // tiles per group; the SH coefficients go through LDS as in k_field_mlp.
 constexpr uint32_t kFeatPitch = 40u;  // halves per LDS feature row (80 bytes)
-template <typename TableT, bool kFromSamples>
+template <typename TableT, bool kFromSamples, bool kFma>
 __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g, const TableT* __restrict__ table, const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, FieldInputs in, uint32_t n_cap,
                                                                    float4* __restrict__ out) {
     const uint32_t n = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
@@ -306,10 +306,10 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
                 put(l, a0, a1);
             }
         };
-        levels_to(n_cell, [&](uint32_t k, float& a0, float& a1) { encode_level_cell<kFromSamples>(in.cells.data + 2ull * in.cells.first[k], p, g.resolution[k], a0, a1); });
-        levels_to(n_dense, [&](uint32_t k, float& a0, float& a1) { encode_level_xpair<TableT, false, kFromSamples>(g, table, p, k, g.resolution[k], true, a0, a1); });
-        levels_to(n_narrow, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFromSamples, false>(g, table, p, k, g.resolution[k], false, a0, a1); });
-        levels_to(16u, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFromSamples>(g, table, p, k, g.resolution[k], false, a0, a1); });
+        levels_to(n_cell, [&](uint32_t k, float& a0, float& a1) { encode_level_cell<kFma>(in.cells.data + 2ull * in.cells.first[k], p, g.resolution[k], a0, a1); });
+        levels_to(n_dense, [&](uint32_t k, float& a0, float& a1) { encode_level_xpair<TableT, false, kFma>(g, table, p, k, g.resolution[k], true, a0, a1); });
+        levels_to(n_narrow, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFma, false>(g, table, p, k, g.resolution[k], false, a0, a1); });
+        levels_to(16u, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFma>(g, table, p, k, g.resolution[k], false, a0, a1); });
         if (in.features_out && s < n) {
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -548,15 +548,16 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
         }
         (void)hipGetLastError();
     }
-#define NERF_FIELD_LAUNCH(K)                                                                                                                   \
-    do {                                                                                                                                       \
-        if (g.table_dtype == NERF_EXT_F32) {                                                                                                   \
-            if (from_samples) K<float, true><<<blocks, kBlockThreads, 0, stream>>>(g, (const float*)table, w.density, w.color, in, n, out4);      \
-            else K<float, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const float*)table, w.density, w.color, in, n, out4);                \
-        } else {                                                                                                                               \
-            if (from_samples) K<half_t, true><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);  \
-            else K<half_t, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);              \
-        }                                                                                                                                      \
+#define NERF_FIELD_LAUNCH(K)                                                                                                                          \
+    do {                                                                                                                                              \
+        if (g.table_dtype == NERF_EXT_F32) {                                                                                                          \
+            if (from_samples) K<float, true, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const float*)table, w.density, w.color, in, n, out4);      \
+            else K<float, false, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const float*)table, w.density, w.color, in, n, out4);                \
+        } else {                                                                                                                                      \
+            if (!from_samples) K<half_t, false, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);  \
+            else if (in.fused_sums) K<half_t, true, true><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4); \
+            else K<half_t, true, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);                \
+        }                                                                                                                                             \
     } while (0)
     if (level_major) NERF_FIELD_LAUNCH(k_field_forward_lv);
     else NERF_FIELD_LAUNCH(k_field_forward);

@@ -987,8 +987,9 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
     // Every field launch of the rounds reads its entries' rays from the round
     // list (qray), so the march writes no per-sample ray index.
     FieldInputs in{};
-    in.samples = R->samples.ptr;
-    in.rays    = R->rays.ptr;
+    in.samples    = R->samples.ptr;
+    in.rays       = R->rays.ptr;
+    in.fused_sums = true;
     for (int a = 0; a < 3; ++a) {  // the field's box is the outermost cascade's
         in.bmin[a] = occ.omin[a];
         in.bmax[a] = occ.omax[a];
@@ -1178,6 +1179,7 @@ NERF_API NerfStatus nerf_ext_render_uniform(NerfExtRenderer* R, const NerfExtMod
     NERF_LAUNCH_CHECK("k_uniform_rays");
     FieldInputs in{};
     in.samples    = R->samples.ptr;
+    in.fused_sums = true;
     in.sample_ray = R->sample_ray.ptr;
     in.rays       = R->rays.ptr;
     for (int a = 0; a < 3; ++a) {

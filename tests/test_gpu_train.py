@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from conftest import announce
-from helpers import L, ext, orc, oracle_grid, assert_rel, assert_adam_step, assert_table_grad, assert_rel_rows, fixed_point_floor
+from helpers import L, ext, orc, DeviceArray, synchronize, byref, oracle_grid, assert_rel, assert_adam_step, assert_table_grad, assert_rel_rows, fixed_point_floor
 
 pytestmark = pytest.mark.gpu
 
@@ -174,6 +174,30 @@ def test_forward_stage(dataset, log2_table):
     want = orc.field_forward(og, table, dp, cp, p, d)
     assert_rel(field[:, 0], want[:, 0], what="sigma", mlp=True)
     assert_rel(field[:, 1:], want[:, 1:], what="rgb", mlp=True)
+
+
+# Dense batches (more than 128 steps per ray) encode inside the field kernel: by
+# tiles up to 2^20 samples of capacity, level by level above.
+@pytest.mark.parametrize("capacity", [1 << 16, (1 << 20) + 64])
+def test_dense_forward_features_equal_encode(dataset, capacity):
+    """A training step encodes a sample to the bits of nerf_ext_encode_forward."""
+    announce(f"train forward stage, dense batch of capacity {capacity}")
+    _, cams, imgs = dataset
+    grid = ext.grid_desc(16, L.NERF_EXT_F16)
+    t = ext.Trainer(grid, imgs.view(np.uint8), cams, occupancy_res=OCC_RES, hyper=ext.hyper_params(loss_scale=LOSS_SCALE), occupancy=ext.occupancy_params(warmup_steps=2, update_interval=4, cells_per_update=OCC_RES ** 3),
+                    initial_rays=RAYS, max_rays=RAYS, sample_capacity=capacity, max_steps_per_ray=200, seed=5, table_init_range=1e-1)
+    t.run_stages(L.NERF_EXT_STAGE_BEGIN, L.NERF_EXT_STAGE_FORWARD)
+    s = _sample_state(t)
+    n = s["stats"].samples
+    assert n > 1 << 14 and not t.buffers().features_lm
+    p, _ = _positions(s)
+    m, _ = t.model()
+    d_p, d_f = DeviceArray.from_numpy(p), DeviceArray((n, 32), np.float16)
+    L.call("nerf_ext_encode_forward", byref(m.grid), m.table, d_p.ptr, n, d_f.ptr, L.NERF_EXT_F16, None)
+    synchronize()
+    got, want = ext.read_device(t.buffers().features, (n, 32), np.uint16), d_f.numpy().view(np.uint16)
+    diff = np.count_nonzero(got != want)
+    assert diff == 0, f"{diff} of {32 * n} features differ"
 
 
 def _composite_oracle(s, field, inv_norm):
