@@ -599,6 +599,8 @@ hipError_t launch_density(const GridParams& g, const void* table, const half_t* 
 constexpr uint32_t kRefFragments = 444u;
 hipError_t ref_pack_weights(const half_t* dparams, const half_t* cparams, half8_t* frags, hipStream_t stream);
 hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_t n, float4* out4, float4* raw4, hipStream_t stream, half_t* dens_out = nullptr);
+// The density network's 16 fp16 outputs alone, [n][16].
+hipError_t launch_ref_density(const half8_t* frags, const FieldInputs& in, uint32_t n, half_t* dens_out, hipStream_t stream);
 // Workgroups, and partials, of the weight-gradient kernels.
 uint32_t ref_grad_blocks(uint32_t np);
 // Training of the reference model (the trainer's stages).  Rows of the
@@ -612,7 +614,7 @@ constexpr uint32_t kRefReduceBlocks = (kRefParams + 255u) / 256u;  // one parame
 constexpr uint32_t kRefMaxSamples = 1u << 20;  // per backward call: the buffers stay below 4 GiB (buffer-descriptor range)
 struct RefTrainLaunch {
     half8_t* frags;    // 64 x kRefFragments
-    half_t* dens;      // [np][16] the forward's density outputs
+    half_t* dens;      // [np][16] density outputs: the forward's, or of launch_ref_density where no forward went before
     half_t* deltas;    // [np][16] their deltas
     float* partial;    // [ref_grad_blocks(np)][kRefParams]
     uint32_t np;       // sample capacity rounded up to 64
@@ -622,9 +624,9 @@ struct RefTrainLaunch {
 // stream: counts = kept, ray and active-ray counts on the device.
 hipError_t launch_ref_composite_train(const RefTrainLaunch& T, const uint32_t* kept, const uint32_t* offsets, const float2* samples, const float4* field, const float4* gt, float4* draw, float* loss_sum,
                                       const uint32_t* n_rays_dev, const uint32_t* n_active_dev, hipStream_t stream);
-// MLP backward (forward recomputed from the sample stream, in.n_dev samples)
-// and the weight gradients x loss_scale into grad [kRefParams] (density then
-// colour), with kRefReduceBlocks squared-norm partials in norm.
+// MLP backward from T.dens and the sample stream (in.n_dev samples): the weight
+// gradients x loss_scale into grad [kRefParams] (density then colour), with
+// kRefReduceBlocks squared-norm partials in norm.
 hipError_t launch_ref_backward_train(const RefTrainLaunch& T, const FieldInputs& in, const float4* draw, float loss_scale, float* grad, double* norm, hipStream_t stream);
 
 // Number of compute units of the current device (cached).

@@ -1489,6 +1489,13 @@ hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_
 
 static_assert(kActRows == kRefActRows && kDltRows == kRefDltRows, "training buffer rows");
 
+hipError_t launch_ref_density(const half8_t* frags, const FieldInputs& in, uint32_t n, half_t* dens_out, hipStream_t stream) {
+    if (n == 0u) return hipSuccess;
+    if (in.samples) k_ref_field<true, true><<<ref_field_blocks(n), kBlockThreads, 0, stream>>>(frags, in, n, nullptr, nullptr, dens_out);
+    else k_ref_field<false, true><<<ref_field_blocks(n), kBlockThreads, 0, stream>>>(frags, in, n, nullptr, nullptr, dens_out);
+    return hipGetLastError();
+}
+
 hipError_t launch_ref_composite_train(const RefTrainLaunch& T, const uint32_t* kept, const uint32_t* offsets, const float2* samples, const float4* field, const float4* gt, float4* draw, float* loss_sum,
                                       const uint32_t* n_rays_dev, const uint32_t* n_active_dev, hipStream_t st) {
     const uint32_t waves = (T.max_rays + kBlockWaves - 1u) / kBlockWaves;
@@ -1579,10 +1586,7 @@ NerfStatus ref_backward(const char* who, const uint16_t* density_params, const u
     in.positions  = positions;
     in.directions = directions;
     hipError_t e  = ref_pack_weights((const half_t*)density_params, (const half_t*)color_params, frags, st);
-    if (e == hipSuccess && !rows) {
-        k_ref_field<false, true><<<ref_field_blocks(n), kBlockThreads, 0, st>>>(frags, in, n, nullptr, nullptr, deltas + 16ull * np);
-        e = hipGetLastError();
-    }
+    if (e == hipSuccess && !rows) e = launch_ref_density(frags, in, n, deltas + 16ull * np, st);
     if (e == hipSuccess && !rows) e = launch_ref_grad<false>(frags, in, n, np, deltas + 16ull * np, (const float4*)draw, loss_scale, deltas, partial, ddensity, dcolor, nullptr, st);
     if (e == hipSuccess && rows) {
         const uint32_t need = np / 64u / kBlockWaves + 1u, cap = device_cu_count() * 2u;

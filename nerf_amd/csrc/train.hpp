@@ -184,8 +184,10 @@ struct StepStreams {
 // first kernel (the occupancy refresh, else the ray pass; hash-grid model)
 // does the begin.  kFoldEnd: the end stage launches nothing and the
 // backward's gradient-norm kernel does the end (before Adam, which reads its
-// own copy of the step index).
-enum : uint32_t { kFoldBegin = 1u, kFoldEnd = 2u };
+// own copy of the step index).  kFoldForward: the same call enqueued the
+// forward, so the reference model's backward starts from its density outputs
+// (a backward enqueued alone computes them from the sample stream).
+enum : uint32_t { kFoldBegin = 1u, kFoldEnd = 2u, kFoldForward = 4u };
 
 // Launches one stage (NERF_EXT_STAGE_*) of a training step on `stream`.
 // `occupancy_update` selects the occupancy-maintenance kernels (the schedule

@@ -2169,7 +2169,10 @@ static hipError_t launch_ref_train_stage(const TrainParams& P, const TrainBuffer
     case NERF_EXT_STAGE_FORWARD: return launch_ref_field(B.ref.frags, in, P.sample_cap, B.field, nullptr, st, B.ref.dens);
     case NERF_EXT_STAGE_COMPOSITE: return launch_ref_composite_train(B.ref, B.kept, B.offsets, B.samples, B.field, B.gt, B.draw, &B.state->loss_sum, &B.state->n_rays, &B.state->n_active, st);
     case NERF_EXT_STAGE_BACKWARD: {
-        const hipError_t e = launch_ref_backward_train(B.ref, in, B.draw, P.loss_scale, B.mlp_grad, B.norm_partials, st);
+        hipError_t e = hipSuccess;
+        if (!(fold & kFoldForward)) e = launch_ref_density(B.ref.frags, in, P.sample_cap, B.ref.dens, st);
+        if (e != hipSuccess) return e;
+        e = launch_ref_backward_train(B.ref, in, B.draw, P.loss_scale, B.mlp_grad, B.norm_partials, st);
         if (e != hipSuccess) return e;
         k_grad_norm<<<1, kNormThreads, 0, st>>>(P, B.norm_partials, norm_partial_count(B), B.state, B.prev, (fold & kFoldEnd) != 0u);
         break;

@@ -44,13 +44,15 @@ bool Trainer::occupancy_due(uint32_t frame) const {
 
 // The fold bits for stage s of a range that starts at `first` and ends at
 // `last` (kFoldBegin: hash-grid model, the range holds the begin and the
-// step's first kernel; kFoldEnd: the range holds the backward and the end).
+// step's first kernel; kFoldEnd: the range holds the backward and the end;
+// kFoldForward: the range holds the forward and the backward).
 uint32_t Trainer::fold_for(uint32_t s, uint32_t first, uint32_t last, bool occ) const {
     uint32_t fold = 0u;
     if (B.model_kind != NERF_EXT_MODEL_REFERENCE && first == NERF_EXT_STAGE_BEGIN && last >= NERF_EXT_STAGE_SAMPLE &&
         (s == NERF_EXT_STAGE_BEGIN || s == (occ ? NERF_EXT_STAGE_OCCUPANCY : NERF_EXT_STAGE_SAMPLE)))
         fold |= kFoldBegin;
     if (first <= NERF_EXT_STAGE_BACKWARD && last == NERF_EXT_STAGE_END && (s == NERF_EXT_STAGE_BACKWARD || s == NERF_EXT_STAGE_END)) fold |= kFoldEnd;
+    if (first <= NERF_EXT_STAGE_FORWARD && s == NERF_EXT_STAGE_BACKWARD) fold |= kFoldForward;
     return fold;
 }
 

@@ -112,6 +112,33 @@ def test_ref_forward_stage(step):
     assert_rel(step["field"], want, rtol=2e-3, what="reference-model field (sigma, rgb) in the trainer", mlp=True, bulk_rtol=1e-3)
 
 
+def test_ref_backward_stage_without_forward(dataset):
+    """The backward needs the samples and the output gradients only: a caller
+    that computes its own field and loss runs it without a forward stage."""
+    announce("reference-model trainer: backward stage alone")
+    t = _trainer(dataset)
+    t.run_stages(L.NERF_EXT_STAGE_BEGIN, L.NERF_EXT_STAGE_BACKWARD)
+    n = t.stats().samples
+    assert n > 1000
+    draw, want = ext.read_device(t.buffers().draw, (n, 4), np.float32), ext.read_device(t.buffers().mlp_grad, (ND + NC,), np.uint32)
+    # The first step's samples and weights again, none of its forward left.
+    u = _trainer(dataset)
+    u.run_stages(L.NERF_EXT_STAGE_BEGIN, L.NERF_EXT_STAGE_SAMPLE)
+    u.synchronize()
+    assert u.stats().samples == n
+    ext.write_device(u.buffers().draw, draw)
+    u.run_stages(L.NERF_EXT_STAGE_BACKWARD, L.NERF_EXT_STAGE_BACKWARD)
+    u.synchronize()
+    got = ext.read_device(u.buffers().mlp_grad, (ND + NC,), np.uint32)
+    assert np.array_equal(got, want), f"{np.count_nonzero(got != want)} gradients differ"
+    # The same step's stages one call each.
+    v = _trainer(dataset)
+    for stage in range(L.NERF_EXT_STAGE_BEGIN, L.NERF_EXT_STAGE_BACKWARD + 1):
+        v.run_stages(stage, stage)
+    v.synchronize()
+    assert np.array_equal(ext.read_device(v.buffers().mlp_grad, (ND + NC,), np.uint32), want)
+
+
 def _raw_from_field(field):
     """The raw outputs that give these activations (softplus sigma with the
     reference's branches, sigmoid rgb), in fp64."""
