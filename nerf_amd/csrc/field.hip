@@ -230,18 +230,20 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, c
 // one 128-byte line per sample where a lane per sample asks for two), which
 // halves the cache lines of the fine levels.
 // What bounds it: the vector-memory path and, beside it, the vector ALUs.
-// The levels run in rolled loops of two (16 unrolled bodies with three paths
+// Renders (kFma) sum their corners with v_fma_mix_f32 (corner_sum).  kRolled:
+// the levels run in rolled loops of two (16 unrolled bodies with three paths
 // each held so many uniform values that 190 of them went through spill lanes,
 // 2,700 vector instructions per group of 64 samples against 2,100), the
-// corner sums of renders take v_fma_mix_f32 (corner_sum), and an incoherent
-// level's entries are fetched as aligned pairs (entry_pair).  Together,
-// 800x800 render 44.4 -> 40.9 ms, three 1280x720 views over five cascades
-// 471 -> 373 ms.
+// leading ones from cell tables, and an incoherent level's entries are fetched
+// as aligned pairs (entry_pair).  Together, 800x800 render 44.4 -> 40.9 ms,
+// three 1280x720 views over five cascades 471 -> 373 ms, before the cell
+// tables.  Unrolled, more of a wave's gathers are in flight, which small
+// launches and scattered points need; launch_field says which goes where.
 // The fp16 features go through LDS (rows of 80 bytes, 16-byte reads of lane
 // group g's levels 4g..4g+3) into the MLP's B-operand layout, four 16-sample
 // tiles per group; the SH coefficients go through LDS as in k_field_mlp.
 constexpr uint32_t kFeatPitch = 40u;  // halves per LDS feature row (80 bytes)
-template <typename TableT, bool kFromSamples, bool kFma>
+template <typename TableT, bool kFromSamples, bool kFma, bool kRolled>
 __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g, const TableT* __restrict__ table, const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, FieldInputs in, uint32_t n_cap,
                                                                    float4* __restrict__ out) {
     const uint32_t n = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
@@ -287,33 +289,47 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
         sh16(d, sh);
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) shl[wv][lane][j] = half4_t{to_half_rne(sh[4u * j]), to_half_rne(sh[4u * j + 1u]), to_half_rne(sh[4u * j + 2u]), to_half_rne(sh[4u * j + 3u])};
-        // Gather: rolled loops over the cell-table, dense and hashed levels
-        // (in that order: resolutions grow with the level), two levels at a
-        // time, features to LDS as they come.
-        auto put = [&](uint32_t l, float a0, float a1) { *reinterpret_cast<half2_t*>(F + lane * kFeatPitch + 2u * l) = half2_t{to_half_rne(a0), to_half_rne(a1)}; };
-        uint32_t l = 0u;
-        auto levels_to = [&](uint32_t end, auto level) {
-            for (; l + 2u <= end; l += 2u) {
-                float a0, a1, b0, b1;
-                level(l, a0, a1);
-                level(l + 1u, b0, b1);
-                put(l, a0, a1);
-                put(l + 1u, b0, b1);
-            }
-            for (; l < end; ++l) {
-                float a0, a1;
-                level(l, a0, a1);
-                put(l, a0, a1);
-            }
-        };
-        levels_to(n_cell, [&](uint32_t k, float& a0, float& a1) { encode_level_cell<kFma>(in.cells.data + 2ull * in.cells.first[k], p, g.resolution[k], a0, a1); });
-        levels_to(n_dense, [&](uint32_t k, float& a0, float& a1) { encode_level_xpair<TableT, false, kFma>(g, table, p, k, g.resolution[k], true, a0, a1); });
-        levels_to(n_narrow, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFma, false>(g, table, p, k, g.resolution[k], false, a0, a1); });
-        levels_to(16u, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFma>(g, table, p, k, g.resolution[k], false, a0, a1); });
-        if (in.features_out && s < n) {
-            __builtin_amdgcn_wave_barrier();
+        if constexpr (kRolled) {
+            // Rolled loops over the cell-table, dense and hashed levels (in that
+            // order: resolutions grow with the level), two levels at a time,
+            // features to LDS as they come.
+            auto put = [&](uint32_t l, float a0, float a1) { *reinterpret_cast<half2_t*>(F + lane * kFeatPitch + 2u * l) = half2_t{to_half_rne(a0), to_half_rne(a1)}; };
+            uint32_t l = 0u;
+            auto levels_to = [&](uint32_t end, auto level) {
+                for (; l + 2u <= end; l += 2u) {
+                    float a0, a1, b0, b1;
+                    level(l, a0, a1);
+                    level(l + 1u, b0, b1);
+                    put(l, a0, a1);
+                    put(l + 1u, b0, b1);
+                }
+                for (; l < end; ++l) {
+                    float a0, a1;
+                    level(l, a0, a1);
+                    put(l, a0, a1);
+                }
+            };
+            levels_to(n_cell, [&](uint32_t k, float& a0, float& a1) { encode_level_cell<kFma>(in.cells.data + 2ull * in.cells.first[k], p, g.resolution[k], a0, a1); });
+            levels_to(n_dense, [&](uint32_t k, float& a0, float& a1) { encode_level_xpair<TableT, false, kFma>(g, table, p, k, g.resolution[k], true, a0, a1); });
+            levels_to(n_narrow, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFma, false>(g, table, p, k, g.resolution[k], false, a0, a1); });
+            levels_to(16u, [&](uint32_t k, float& a0, float& a1) { encode_level_lanepair<TableT, kFma>(g, table, p, k, g.resolution[k], false, a0, a1); });
+        } else {
+            // Four levels per 16-byte LDS store.
 #pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) *reinterpret_cast<half8_t*>(in.features_out + (uint64_t)s * 32u + 8u * k) = *reinterpret_cast<const half8_t*>(F + lane * kFeatPitch + 8u * k);
+            for (uint32_t k = 0; k < 4u; ++k) {
+                half8_t h;
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j) {
+                    const uint32_t l = 4u * k + j;
+                    float a0, a1;
+                    if (g.dense[l] != 0u) encode_level_xpair<TableT, false, kFma>(g, table, p, l, g.resolution[l], true, a0, a1);
+                    else encode_level_lanepair<TableT, kFma, false>(g, table, p, l, g.resolution[l], false, a0, a1);
+                    h[2u * j]      = to_half_rne(a0);
+                    h[2u * j + 1u] = to_half_rne(a1);
+                }
+                *reinterpret_cast<half8_t*>(F + lane * kFeatPitch + 8u * k) = h;
+                if (in.features_out && s < n) *reinterpret_cast<half8_t*>(in.features_out + (uint64_t)s * 32u + 8u * k) = h;
+            }
         }
         __builtin_amdgcn_wave_barrier();  // LDS traffic of one wave completes in order
         float v[4];
@@ -548,19 +564,24 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
         }
         (void)hipGetLastError();
     }
-#define NERF_FIELD_LAUNCH(K)                                                                                                                          \
-    do {                                                                                                                                              \
-        if (g.table_dtype == NERF_EXT_F32) {                                                                                                          \
-            if (from_samples) K<float, true, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const float*)table, w.density, w.color, in, n, out4);      \
-            else K<float, false, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const float*)table, w.density, w.color, in, n, out4);                \
-        } else {                                                                                                                                      \
-            if (!from_samples) K<half_t, false, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);  \
-            else if (in.fused_sums) K<half_t, true, true><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4); \
-            else K<half_t, true, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);                \
-        }                                                                                                                                             \
+    // Gather of the level-major kernel: rolled loops for the large renders (those
+    // with cell tables) and for renders from tables of at most 8 MiB; unrolled
+    // for the rest.  Rolled against unrolled: 200x150 pixels at 400 steps,
+    // T = 2^17, 933 / 965 us; 160x120 at 512, T = 2^18, 711 / 701; 400x300 at 64,
+    // T = 2^19, 1,437 / 1,416; 2^20 + 1 random points at T = 2^19, 585 / 552, 2^21
+    // 1,210 / 1,158; an fp32 table, 128x96 at 400, 500 / 483.
+    const bool rolled = in.fused_sums && g.table_dtype == NERF_EXT_F16 && (in.cells.levels != 0u || g.table_size <= (1u << 17));
+#define NERF_FIELD_LAUNCH(TABLE, ...)                                                                                                                                      \
+    do {                                                                                                                                                                   \
+        if (level_major) k_field_forward_lv<TABLE, __VA_ARGS__, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const TABLE*)table, w.density, w.color, in, n, out4);         \
+        else k_field_forward<TABLE, __VA_ARGS__><<<blocks, kBlockThreads, 0, stream>>>(g, (const TABLE*)table, w.density, w.color, in, n, out4);                             \
     } while (0)
-    if (level_major) NERF_FIELD_LAUNCH(k_field_forward_lv);
-    else NERF_FIELD_LAUNCH(k_field_forward);
+    if (level_major && rolled) k_field_forward_lv<half_t, true, true, true><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, in, n, out4);
+    else if (g.table_dtype == NERF_EXT_F32 && from_samples) NERF_FIELD_LAUNCH(float, true, false);
+    else if (g.table_dtype == NERF_EXT_F32) NERF_FIELD_LAUNCH(float, false, false);
+    else if (!from_samples) NERF_FIELD_LAUNCH(half_t, false, false);
+    else if (in.fused_sums) NERF_FIELD_LAUNCH(half_t, true, true);
+    else NERF_FIELD_LAUNCH(half_t, true, false);
 #undef NERF_FIELD_LAUNCH
     return hipGetLastError();
 }

@@ -150,3 +150,25 @@ def test_render_with_cell_tables_matches_hash_table(log2_t, finest, width, heigh
         synchronize()
         outs.append((rgba.numpy(), rgb.numpy().view(np.uint32)))
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+
+
+# Twelve million possible samples, no cell tables: an fp32 table and an
+# fp16 one of either gather (T = 2^17, 2^18), and one whose render takes the tile
+# kernel (T = 2^19).  The same images from counted chunks of more than 2^20
+# samples (level-major) and of at most 2^19 (tiles).
+@pytest.mark.parametrize("dtype,log2_t,width,height", [(L.NERF_EXT_F32, 15, 130, 90), (L.NERF_EXT_F16, 17, 131, 89), (L.NERF_EXT_F16, 18, 128, 93), (L.NERF_EXT_F16, 19, 133, 88)])
+def test_render_is_the_same_from_every_field_kernel(dtype, log2_t, width, height):
+    announce(f"render {width}x{height} at 1024 steps, T=2^{log2_t}, dtype {dtype}: default, counted chunks")
+    _, bits = _scene_setup()
+    model = ext.Model.create(ext.grid_desc(log2_t, dtype), seed=4, table_range=1.0)
+    cams = [ext.camera_orbit(0, 3, 1.32, CENTRE, width, height, 1111.0 * width / 800.0)]
+    occ = ext.occupancy_struct(bits, 128)
+    outs = []
+    for chunk in (0, 1 << 29, 1 << 19):
+        rgb = DeviceArray((1, height, width, 3), np.float32)
+        rgba, stats = ext.Renderer().render(model, occ, cams, 1024, rgb=rgb, chunk_samples=chunk, timed=True)
+        synchronize()
+        assert stats.samples > 1 << 20
+        outs.append((rgba.numpy(), rgb.numpy().view(np.uint32)))
+    for other in outs[1:]:
+        assert np.array_equal(outs[0][0], other[0]) and np.array_equal(outs[0][1], other[1])
