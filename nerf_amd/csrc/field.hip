@@ -515,17 +515,25 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
     // Renders and other large launches take the level-major kernel, 3
     // workgroups per CU (its LDS and register budget); small ones the tile
     // kernel, whose 16-sample tiles leave a shorter tail when a launch is only
-    // a few rounds of work (2^18 training samples: 67 vs 93 us).  A render
-    // round's n is its capacity, of which it fills about a third: 100x75
-    // pixels at 256 steps (1.9 M entries) 274 us per render with tiles, 284
-    // level-major; 160x120 at 512 (9.8 M) 865 / 882; 200x150 at 512 (15.4 M)
-    // 1,458 / 1,441.  The tile kernel runs 4 workgroups per CU: 2^18 samples
-    // are 16,384 tiles, exactly 4 per wave (67 us; 3 per CU leave 5 or 6 tiles
-    // per wave, 71 us; 5 and 6 per CU, 77 us).  The level-major kernel
-    // measured slower with 8-wave workgroups at 4 waves per SIMD (52.5 vs
-    // 49.8 ms per 800x800 render: more waves than its L1 serves) and with 4
-    // workgroups per CU (100x75: 295 vs 284 us).
-    const bool level_major  = n > (in.sample_index ? 3u << 22 : 1u << 20);
+    // a few rounds of work (2^18 training samples: 67 vs 93 us).  The tile
+    // kernel runs 4 workgroups per CU: 2^18 samples are 16,384 tiles, exactly
+    // 4 per wave (67 us; 3 per CU leave 5 or 6 tiles per wave, 71 us; 5 and 6
+    // per CU, 77 us).  The level-major kernel measured slower with 8-wave
+    // workgroups at 4 waves per SIMD (52.5 vs 49.8 ms per 800x800 render: more
+    // waves than its L1 serves) and with 4 workgroups per CU (100x75: 295 vs
+    // 284 us).
+    // A slot render's n is its capacity, of which it fills about a third, and
+    // its lanes share lines on the narrow levels only: without cell tables (below
+    // 2^24 entries) it takes tiles when the table exceeds 16 MiB and it is short
+    // or has at most six narrow levels.  Whole renders, tiles against level-major
+    // (five scenes each): T = 2^19, 100x75 at 256 steps 0.94-1.01, 160x120 at 512
+    // 0.91-0.98, 176x92 at 1,000 0.92-0.97; T = 2^20, 80x45 over five cascades
+    // 0.93-0.98; but over five cascades at 120x68 (eleven narrow levels)
+    // 1.06-1.11, 300x200 at 64 (seven) 1.00-1.02, T = 2^18 160x120 at 512 1.03
+    // and T = 2^17 1.09-1.12.  Chunks planned from counts are full: 800x600 in
+    // chunks of 6 x 2^20 samples 37.5 / 35.1 ms.
+    const bool tiles       = in.slot_rays && g.table_dtype == NERF_EXT_F16 && g.table_size >= (1u << 19) && n < (1u << 24) && (n <= (1u << 21) || in.narrow_end <= 6u);
+    const bool level_major = n > (1u << 20) && !tiles;
     const uint32_t blocks   = (persistent_blocks(n, level_major ? 3u : 4u) + 7u) / 8u * 8u;  // whole XCD rounds
     const bool from_samples = in.samples != nullptr;
     if (in.sparse && from_samples && in.features_out && !in.sample_index && !in.alpha_in_order && g.table_dtype != NERF_EXT_F32 && g.n_levels == 16u) {
