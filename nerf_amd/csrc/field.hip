@@ -170,6 +170,25 @@ __global__ __launch_bounds__(kBlockThreads) void k_density_forward(GridParams g,
     }
 }
 
+// Whether an array's points are scattered: at how many of the sixteen levels
+// neighbouring points (32 pairs over the array, one workgroup of 256) find
+// their first corner in one 128-byte line, on average.  Uniform random points
+// share none, points along rays of 64, 256 and 1,024 samples 4, 8 and 12, a
+// lattice or a march's order 11-14.  Split against fused, T = 2^17: 300,007
+// points 8 levels 91 / 75 us, 4 levels 96 / 98; T = 2^19: 12 levels 61 / 53, 8
+// levels 75 / 119.
+__device__ bool points_scattered(const GridParams& g, const float* __restrict__ pos, uint32_t n) {
+    const uint32_t level = threadIdx.x & 15u, N = g.resolution[level];
+    const bool dense     = g.dense[level] != 0u;
+    int shared           = 0;
+    for (uint32_t pair = threadIdx.x >> 4; pair < 32u; pair += 16u) {  // uniform: two turns
+        const float* p = pos + 3ull * ((uint64_t)pair * (n - 2u) / 31u);
+        const uint32_t a = corner_index(level_cell(p, N), 0u, N, dense, g.table_size - 1u), b = corner_index(level_cell(p + 3, N), 0u, N, dense, g.table_size - 1u);
+        shared += __syncthreads_count((a >> 5) == (b >> 5));
+    }
+    return shared < 32 * (g.table_size > (1u << 17) ? 10 : 6);
+}
+
 // Full field: sigma, rgb per sample.  Inputs either explicit (positions,
 // directions) or march samples (t_mid, dt, ray) with per-ray o, d.  The
 // weight fragments stay in LDS (84 VGPRs instead of 157): on a training
@@ -179,6 +198,13 @@ __global__ __launch_bounds__(kBlockThreads) void k_density_forward(GridParams g,
 template <typename TableT, bool kFromSamples, bool kFma>
 __global__ __launch_bounds__(kBlockThreads) void k_field_forward(GridParams g, const TableT* __restrict__ table, const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, FieldInputs in, uint32_t n_cap, float4* __restrict__ out) {
     const uint32_t n = in.n_dev ? min(*in.n_dev, n_cap) : n_cap;
+    if constexpr (!kFromSamples) {
+        if (in.scattered) {
+            const bool scattered = points_scattered(g, in.positions, n);
+            if (blockIdx.x == 0u && threadIdx.x == 0u) *in.scattered = scattered ? 1u : 0u;
+            if (scattered) return;
+        }
+    }
     __shared__ __align__(16) half8_t frag[kFieldFrags][kWaveSize];
     const uint32_t lane = threadIdx.x & 63u, grp = lane >> 4, s16 = lane & 15u;
     for (uint32_t f = threadIdx.x >> 6; f < kFieldFrags; f += kBlockWaves) frag[f][lane] = mlp_fragment(dparams, cparams, f, lane);
@@ -375,7 +401,8 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
 struct DirsFromArray {
     const float* dirs;
     uint32_t n;
-    __device__ __forceinline__ uint32_t count() const { return n; }
+    const uint32_t* gate = nullptr;  // optional device word; nothing to do where it holds 0
+    __device__ __forceinline__ uint32_t count() const { return gate && *gate == 0u ? 0u : n; }
     __device__ __forceinline__ void at(uint32_t q, float d[3]) const {
 #pragma unroll
         for (int a = 0; a < 3; ++a) d[a] = dirs[3ull * q + a];
@@ -417,6 +444,7 @@ template <typename Dirs, typename Feats>
 __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(kMlpWaves, 8))) void k_field_mlp(const half_t* __restrict__ dparams, const half_t* __restrict__ cparams, Feats features,
                                                                                                                   Dirs dirs, float4* __restrict__ out) {
     const uint32_t n = dirs.count();
+    if (n == 0u) return;
     __shared__ __align__(16) half8_t frag[kFieldFrags][kWaveSize];
     __shared__ half4_t shl[kBlockWaves][kGroupSamples][4];
     const uint32_t lane = threadIdx.x & 63u, grp = lane >> 4, s16 = lane & 15u, wv = threadIdx.x >> 6;
@@ -548,23 +576,40 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
             k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromRows{in.features_out}, dirs, out4);
         return hipGetLastError();
     }
-    // Points from an array, which may lie anywhere (a wave's gathers then share
-    // no lines, and all levels together do not fit an XCD's L2): encoded level
-    // group by level group, then the MLPs over the features, when that is
-    // faster.  Random points, fused against split: T = 2^19: 2^14 points 17.6
-    // / 20.6 us, 2^16 53 / 31, 300,007 222 / 109, 2^20 710 / 350; T = 2^17:
-    // 2^16 36 / 30, 2^20 377 / 306; T = 2^15: 2^16 30 / 28, 2^20 269 / 279.
-    // (Points in march order measure the same either way up to 2^20, and much
-    // faster in the level-major kernel beyond, 0.1 against 0.35 ns each, which
-    // therefore keeps the larger arrays.)  The fused kernel needs no memory: a
-    // stream under capture and a failed allocation take it.
-    if (!from_samples && !in.n_dev && !in.features_out && g.table_dtype == NERF_EXT_F16 && g.n_levels == 16u && n <= (1u << 20) && n >= (g.table_size > (1u << 17) ? 1u << 15 : 1u << 16) && g.table_size >= (1u << 17)) {
+    // Points from an array may lie anywhere: a wave's gathers then share no
+    // lines, and all levels together do not fit an XCD's L2.  Such arrays are
+    // encoded level group by level group, then the MLPs run over the features.
+    // Fused against split, random points: T = 2^19: 2^15 21 / 24 us (the launches'
+    // host time), 2^16 47 / 30, 81,920 78 / 36, 300,007 216 / 99, 2^20 709 / 308;
+    // T = 2^17: 131,072 53 / 47, 300,007 120 / 96, 2^20 375 / 297; T = 2^15: 2^20
+    // 269 / 279.  Lattices and points in march order share lines in the fused
+    // kernel: T = 2^17, 300,007: 50 / 66-73; 2^18 to 2^20 up to 2^19 points: within
+    // 10 us either way (2^16: 17-28 / 24-28); 2^20 at T = 2^19: 132-163 / 143-176,
+    // at T = 2^21: 141-189 / 203-262.  So small arrays stay fused, and where
+    // much is at stake the tile kernel first looks at the points and does its work
+    // or leaves it to the other two launches: 5 us for scattered points, 7-10 us
+    // for ordered ones (2^20, T = 2^21: random 542, march order 151, lattice 183).
+    // More than 2^20 points take the level-major kernel whatever their order
+    // (march order 0.1 ns each, random points 0.55 at T = 2^19).  The fused
+    // kernels need no memory: a stream under capture and a failed allocation take
+    // them.
+    const bool small_table = g.table_size <= (1u << 17);
+    if (!from_samples && !in.n_dev && !in.features_out && g.table_dtype == NERF_EXT_F16 && g.n_levels == 16u && g.table_size >= (1u << 17) && n <= (1u << 20) && n > (small_table ? 3u << 16 : 1u << 16)) {
+        const bool look = n > (1u << 19) || (n > (3u << 16) && (small_table || g.table_size >= (1u << 21)));
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        uint32_t* lm                   = nullptr;
-        if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone && scratch_alloc((void**)&lm, 64ull * n, stream) == hipSuccess) {
-            hipError_t e = launch_encode_positions(g, (const half_t*)table, in.positions, n, lm, stream);
+        uint32_t* lm                   = nullptr;  // features [16][n], then the gate
+        if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone && scratch_alloc((void**)&lm, 64ull * n + 4u, stream) == hipSuccess) {
+            uint32_t* gate = look ? lm + 16ull * n : nullptr;
+            hipError_t e   = hipSuccess;
+            if (gate) {
+                FieldInputs v = in;
+                v.scattered   = gate;
+                k_field_forward<half_t, false, false><<<blocks, kBlockThreads, 0, stream>>>(g, (const half_t*)table, w.density, w.color, v, n, out4);
+                e = hipGetLastError();
+            }
+            if (e == hipSuccess) e = launch_encode_positions(g, (const half_t*)table, in.positions, n, gate, lm, stream);
             if (e == hipSuccess) {
-                k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromLevels{lm, n}, DirsFromArray{in.directions, n}, out4);
+                k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromLevels{lm, n}, DirsFromArray{in.directions, n, gate}, out4);
                 e = hipGetLastError();
             }
             const hipError_t f = hipFreeAsync(lm, stream);

@@ -249,12 +249,15 @@ hipError_t build_cell_tables(const GridParams& g, const half_t* table, const Cel
 
 namespace {
 
+// most: 256-point blocks per level group that get a workgroup of their own;
+// beyond, each takes several.
 template <typename Points>
-hipError_t launch_encode_split(const GridParams& g, const half_t* table, const Points& src, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream) {
+hipError_t launch_encode_split(const GridParams& g, const half_t* table, const Points& src, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream, uint32_t most = 0xFFFFFFFFu) {
     if (cap == 0u) return hipSuccess;
     if (g.n_levels != 16u || g.table_dtype != NERF_EXT_F16) return hipErrorInvalidValue;
     const uint64_t level_bytes = (uint64_t)g.table_size * g.n_features * 2u;
-    const uint32_t blocks_256  = (cap + 255u) / 256u;
+    const uint32_t all_blocks = (cap + 255u) / 256u, turns = all_blocks / most + (all_blocks % most ? 1u : 0u);
+    const uint32_t blocks_256 = (all_blocks + turns - 1u) / turns;
     // Four levels per XCD when four fit in half of its L2; else one level per
     // XCD in two phases (levels 0-7, then 8-15; one launch whose second half
     // of workgroups, dispatched after the first, takes the second phase):
@@ -279,8 +282,10 @@ hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const
     return launch_encode_split(g, table, PointsFromSamples{in.samples, in.sample_ray, in.rays, in.n_dev, cap, {in.bmin[0], in.bmin[1], in.bmin[2]}, {in.bmax[0], in.bmax[1], in.bmax[2]}}, cap, features, lm, stream);
 }
 
-hipError_t launch_encode_positions(const GridParams& g, const half_t* table, const float* positions, uint32_t n, uint32_t* lm, hipStream_t stream) {
-    return launch_encode_split(g, table, PointsFromArray{positions, n}, n, nullptr, lm, stream);
+hipError_t launch_encode_positions(const GridParams& g, const half_t* table, const float* positions, uint32_t n, const uint32_t* gate, uint32_t* lm, hipStream_t stream) {
+    // Gated, the workgroups may have nothing to do: 65,536 of them (2^20 points)
+    // take 18 us to end, 16,384 8 us, and with work 309 -> 314 us.
+    return launch_encode_split(g, table, PointsFromArray{positions, n, gate}, n, nullptr, lm, stream, gate ? 1024u : 0xFFFFFFFFu);
 }
 
 }  // namespace nerf_hip

@@ -161,15 +161,28 @@ def test_split_encode_then_mlp_equals_fused_field(log2_t):
     assert diff == 0, f"{diff} of {4 * n} values differ"
 
 
-# Point arrays of 2^15 (2^16 at T = 2^17) to 2^20 points take the level-split
-# encode and the MLP pass, smaller ones the fused kernel: both limits, ragged
-# counts, one and four levels per XCD.
-@pytest.mark.parametrize("log2_t,n", [(17, 1 << 16), (17, (1 << 16) + 77), (18, 1 << 15), (19, (1 << 15) + 1), (20, 40007), (19, 1 << 20)])
-def test_field_forward_split_equals_fused(log2_t, n):
-    announce(f"field forward by level split against the fused kernel, T=2^{log2_t}, n={n}")
+# Point arrays of more than 2^16 (3 x 2^16 at T = 2^17) and up to 2^20 points take
+# the level-split encode and the MLP pass, smaller ones the fused kernel.  Above
+# 2^19 points (3 x 2^16 at T = 2^17 and from 2^21 on) the device looks at the
+# points first and leaves ordered ones to the fused kernel.  Both sides of the
+# limits, ragged counts, one and four levels per XCD; random points, rays of 64
+# (scattered), 256 (either) and 1,024 samples, a lattice; non-finite coordinates
+# at the ends of the array, which the look reads.
+@pytest.mark.parametrize("log2_t,n,order", [(17, 1 << 16, 0), (17, (1 << 16) + 77, 0), (18, 1 << 15, 0), (18, (1 << 16) + 1, 0), (19, (1 << 15) + 1, 0), (20, 40007, 0), (19, 1 << 20, 0), (21, 100003, 0),
+                                             (17, 3 << 16, 0), (17, 200001, 0), (17, 200001, 256), (17, 200001, 1024), (18, 70001, 64), (18, 600011, 64), (19, 600011, 256), (20, 1 << 20, 1024), (21, 196609, -1), (21, 300007, 0)])
+def test_field_forward_split_equals_fused(log2_t, n, order):
+    announce(f"field forward by level split against the fused kernel, T=2^{log2_t}, n={n}, order {order}")
     desc = ext.grid_desc(log2_t, L.NERF_EXT_F16)
     model = ext.Model.create(desc, seed=6, table_range=1.0)
     pos, dirs = points(n, seed=31), unit_dirs(n, seed=32)
+    if order > 0:  # that many samples along each segment between two random points
+        i = np.arange(n)
+        ends, t = points(2 * (n // order + 1), seed=33).reshape(-1, 2, 3)[i // order], ((i % order + 0.5) / order)[:, None]
+        pos = (ends[:, 0] + t * (ends[:, 1] - ends[:, 0])).astype(np.float32)
+    elif order < 0:  # a lattice, x fastest
+        i, side = np.arange(n), round(n ** (1 / 3)) + 1
+        pos = (np.stack([i % side, i // side % side, i // side // side], 1) / side).astype(np.float32)
+    pos[0], pos[-1] = np.nan, np.inf
     d_pos, d_dir, d_o, d_f = DeviceArray.from_numpy(pos), DeviceArray.from_numpy(dirs), DeviceArray((n, 4), np.float32), DeviceArray((n, 4), np.float32)
     ms = model.struct()
     L.call("nerf_ext_field_forward", byref(ms), d_pos.ptr, d_dir.ptr, n, d_o.ptr, None)
