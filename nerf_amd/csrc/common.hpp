@@ -563,18 +563,23 @@ struct PointsFromSamples {
 // Point sources of the XCD-split encode (hashgrid.hip): positions in the
 // grid's unit cube from an array, or from a march sample stream (FieldInputs
 // mode B, the same operations as the field kernels use).
-// gate: optional device word; no points where it holds 0.
 struct PointsFromArray {
     const float* pos;
     uint32_t n;
-    const uint32_t* gate = nullptr;
-    __device__ __forceinline__ uint32_t count() const { return gate && *gate == 0u ? 0u : n; }
+    __device__ __forceinline__ uint32_t count() const { return n; }
     __device__ __forceinline__ void at(uint32_t i, float x[3]) const {
         const float3 p = *reinterpret_cast<const float3*>(pos + 3ull * i);
         x[0]           = p.x;
         x[1]           = p.y;
         x[2]           = p.z;
     }
+};
+
+// A source whose points are there only where a device word is not 0.
+template <typename Source>
+struct Gated : Source {
+    const uint32_t* gate;
+    __device__ __forceinline__ uint32_t count() const { return *gate ? Source::count() : 0u; }
 };
 
 struct FieldWeights {
@@ -587,8 +592,8 @@ struct FieldWeights {
 // Level-split encode of a march sample stream: features [cap][32] fp16 rows,
 // or with lm, level-major fp16 pairs lm[level * cap + sample].
 hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const FieldInputs& in, uint32_t cap, half_t* features, uint32_t* lm, hipStream_t stream);
-// The same for an array of points in the unit cube, level-major; nothing where
-// *gate is 0.
+// The same for an array of points in the unit cube, level-major; with a gate,
+// nothing where *gate is 0.
 hipError_t launch_encode_positions(const GridParams& g, const half_t* table, const float* positions, uint32_t n, const uint32_t* gate, uint32_t* lm, hipStream_t stream);
 // Fills the cell tables of levels [0, t.levels) from the hash table (fp16).
 hipError_t build_cell_tables(const GridParams& g, const half_t* table, const CellTables& t, hipStream_t stream);

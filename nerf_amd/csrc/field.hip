@@ -401,8 +401,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_field_forward_lv(GridParams g
 struct DirsFromArray {
     const float* dirs;
     uint32_t n;
-    const uint32_t* gate = nullptr;  // optional device word; nothing to do where it holds 0
-    __device__ __forceinline__ uint32_t count() const { return gate && *gate == 0u ? 0u : n; }
+    __device__ __forceinline__ uint32_t count() const { return n; }
     __device__ __forceinline__ void at(uint32_t q, float d[3]) const {
 #pragma unroll
         for (int a = 0; a < 3; ++a) d[a] = dirs[3ull * q + a];
@@ -609,7 +608,9 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
             }
             if (e == hipSuccess) e = launch_encode_positions(g, (const half_t*)table, in.positions, n, gate, lm, stream);
             if (e == hipSuccess) {
-                k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromLevels{lm, n}, DirsFromArray{in.directions, n, gate}, out4);
+                const DirsFromArray dirs{in.directions, n};
+                if (gate) k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromLevels{lm, n}, Gated<DirsFromArray>{dirs, gate}, out4);
+                else k_field_mlp<<<mlp_pass_blocks(n), kBlockThreads, 0, stream>>>(w.density, w.color, FeatsFromLevels{lm, n}, dirs, out4);
                 e = hipGetLastError();
             }
             const hipError_t f = hipFreeAsync(lm, stream);

@@ -285,7 +285,8 @@ hipError_t launch_encode_samples(const GridParams& g, const half_t* table, const
 hipError_t launch_encode_positions(const GridParams& g, const half_t* table, const float* positions, uint32_t n, const uint32_t* gate, uint32_t* lm, hipStream_t stream) {
     // Gated, the workgroups may have nothing to do: 65,536 of them (2^20 points)
     // take 18 us to end, 16,384 8 us, and with work 309 -> 314 us.
-    return launch_encode_split(g, table, PointsFromArray{positions, n, gate}, n, nullptr, lm, stream, gate ? 1024u : 0xFFFFFFFFu);
+    if (gate) return launch_encode_split(g, table, Gated<PointsFromArray>{{positions, n}, gate}, n, nullptr, lm, stream, 1024u);
+    return launch_encode_split(g, table, PointsFromArray{positions, n}, n, nullptr, lm, stream);
 }
 
 }  // namespace nerf_hip
