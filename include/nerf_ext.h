@@ -134,8 +134,11 @@ typedef struct NerfExtModel {
 
 /* Full field at points with view directions: out [n][4] = (sigma, r, g, b),
  * sigma = exp(density raw 0), rgb = sigmoid(colour raw 0..2); positions in
- * the unit cube of the grid.  A model of kind NERF_EXT_MODEL_REFERENCE runs
- * nerf_ext_ref_field_forward instead (world positions, softplus sigma). */
+ * the unit cube of the grid.  Arrays of 65,537 to 2^20 points use up to 64 MiB
+ * of temporary device memory on the stream where that is faster; without it, and
+ * on a stream under capture, one kernel that needs none gives the same bits.  A
+ * model of kind NERF_EXT_MODEL_REFERENCE runs nerf_ext_ref_field_forward instead
+ * (world positions, softplus sigma). */
 NERF_API NerfStatus nerf_ext_field_forward(const NerfExtModel* model, const float* positions, const float* directions, uint32_t n, float* out, void* stream);
 /* Reference-model mode: the reference's own network (backend-cuda.cu:23-54).
  * Frequency encoding of the world position (10 levels) and of the direction
@@ -144,7 +147,9 @@ NERF_API NerfStatus nerf_ext_field_forward(const NerfExtModel* model, const floa
  * (3 used) (:918-943); fp16 weights packed [out][in], input layer first
  * (:828-834, :1213-1241).  out [n][4] = (softplus(raw density 0), sigmoid of
  * raw colour 0..2) (:909-917); raw (optional) [n][4] = the fp16-rounded raw
- * outputs.  Init: :1810-1847 on these shapes. */
+ * outputs.  Init: :1810-1847 on these shapes.  The point calls of this network
+ * (nerf_ext_ref_field_forward, nerf_ext_ref_backward and _rows) use temporary
+ * device memory and are refused on a stream under capture. */
 NERF_API NerfStatus nerf_ext_ref_mlp_init(uint32_t network /* 0 density, 1 colour */, float* params_host);
 NERF_API NerfStatus nerf_ext_ref_field_forward(const uint16_t* density_params, const uint16_t* color_params, const float* positions, const float* directions, uint32_t n, float* out, float* raw, void* stream);
 /* Composite forward + backward with the reference's loss (backend-cuda.cu

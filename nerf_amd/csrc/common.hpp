@@ -649,7 +649,10 @@ uint32_t device_cu_count();
 // back to the system at the next synchronisation and the call after that
 // allocates anew.  scratch_trim gives the current GPU's unused blocks back;
 // the destroy calls of the library's objects do, and an allocation that fails
-// does before it is tried once more.  Safe from any thread, for any stream.
+// does before it is tried once more.  Where the pool cannot be made the default
+// one serves.  Refused on a stream under capture: a graph that held the
+// allocation, replayed between eager calls, faulted the GPU.  Safe from any
+// thread, for any stream.
 constexpr uint64_t kScratchKept = 192ull << 20;
 hipError_t scratch_alloc(void** p, uint64_t bytes, hipStream_t stream);
 void scratch_trim();

@@ -595,9 +595,8 @@ hipError_t launch_field(const GridParams& g, const void* table, const FieldWeigh
     const bool small_table = g.table_size <= (1u << 17);
     if (!from_samples && !in.n_dev && !in.features_out && g.table_dtype == NERF_EXT_F16 && g.n_levels == 16u && g.table_size >= (1u << 17) && n <= (1u << 20) && n > (small_table ? 3u << 16 : 1u << 16)) {
         const bool look = n > (1u << 19) || (n > (3u << 16) && (small_table || g.table_size >= (1u << 21)));
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        uint32_t* lm                   = nullptr;  // features [16][n], then the gate
-        if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone && scratch_alloc((void**)&lm, 64ull * n + 4u, stream) == hipSuccess) {
+        uint32_t* lm = nullptr;  // features [16][n], then the gate
+        if (scratch_alloc((void**)&lm, 64ull * n + 4u, stream) == hipSuccess) {
             uint32_t* gate = look ? lm + 16ull * n : nullptr;
             hipError_t e   = hipSuccess;
             if (gate) {

@@ -54,13 +54,18 @@ hipError_t scratch_pool(bool create, hipMemPool_t* out) {
         props.handleTypes   = hipMemHandleTypeNone;
         props.location.type = hipMemLocationTypeDevice;
         props.location.id   = dev;
-        hipMemPool_t pool   = nullptr;
-        e                   = hipMemPoolCreate(&pool, &props);
+        // Relaxed: a capture that another thread has under way forbids the
+        // creation otherwise, and is broken by the attempt.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        e                         = hipThreadExchangeStreamCaptureMode(&mode);
         if (e != hipSuccess) return e;
-        uint64_t kept = kScratchKept;
-        e             = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &kept);
+        hipMemPool_t pool = nullptr;
+        e                 = hipMemPoolCreate(&pool, &props);
+        uint64_t kept     = kScratchKept;
+        if (e == hipSuccess) e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &kept);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (e != hipSuccess) {
-            (void)hipMemPoolDestroy(pool);
+            if (pool) (void)hipMemPoolDestroy(pool);
             return e;
         }
         g_scratch_pool[dev] = pool;
@@ -72,9 +77,15 @@ hipError_t scratch_pool(bool create, hipMemPool_t* out) {
 }  // namespace
 
 hipError_t scratch_alloc(void** p, uint64_t bytes, hipStream_t stream) {
-    hipMemPool_t pool = nullptr;
-    hipError_t e      = scratch_pool(true, &pool);
+    hipMemPool_t pool              = nullptr;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipError_t e                   = hipStreamIsCapturing(stream, &capture);
+    if (e == hipSuccess && capture != hipStreamCaptureStatusNone) e = hipErrorStreamCaptureUnsupported;
     if (e != hipSuccess) return e;
+    if (scratch_pool(true, &pool) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipMallocAsync(p, bytes, stream);
+    }
     e = hipMallocFromPoolAsync(p, bytes, pool, stream);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
