@@ -645,6 +645,16 @@ struct NerfExtRenderer {
             cap = 0;
         }
     };
+    // A buffer that the render cannot do without.  Where memory is short the
+    // tables that an earlier render left go first.
+    template <typename T>
+    hipError_t need(Buf<T>& b, uint64_t n) {
+        const hipError_t e = b.reserve(n);
+        if (e != hipErrorOutOfMemory || !cells.ptr) return e;
+        (void)hipGetLastError();
+        cells.release();
+        return b.reserve(n);
+    }
     Buf<NerfExtCamera> cams;
     Buf<float4> rays;
     Buf<uint32_t> counts, offsets, scan_tmp;
@@ -769,7 +779,9 @@ uint32_t narrow_levels(const GridParams& g, const NerfExtCamera* cams, uint32_t 
 // a third to a half of the possible samples are marched, and an early stop
 // leaves fewer.  Renders of fewer than 2^24 possible samples gain less than
 // the extra launch costs (100x75 at 256 steps: 299 -> 304 us).  Without
-// memory for the tables the render reads the hash table.
+// memory for the tables the render reads the hash table; they are kept for the
+// next render until the renderer is destroyed or another of its buffers needs
+// the memory.
 constexpr uint64_t kCellMinSamples = 1ull << 24;
 constexpr uint64_t kCellMax        = 1ull << 26;  // cells of all tables (32 bytes each)
 constexpr uint32_t kCellMaxRes     = 511u;        // a level's table stays below 4 GiB (32-bit offsets)
@@ -912,12 +924,12 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
     const uint32_t n_rays = (uint32_t)n64;
     hipStream_t st        = (hipStream_t)d->stream;
 
-    NERF_HIP_TRY(R->cams.reserve(d->view_count));
-    NERF_HIP_TRY(R->rays.reserve(2ull * n_rays));
-    NERF_HIP_TRY(R->counts.reserve(n_rays));
-    NERF_HIP_TRY(R->offsets.reserve(n_rays));
-    NERF_HIP_TRY(R->scan_tmp.reserve(scan_tmp_words(n_rays)));
-    NERF_HIP_TRY(R->total.reserve(1));
+    NERF_HIP_TRY(R->need(R->cams, d->view_count));
+    NERF_HIP_TRY(R->need(R->rays, 2ull * n_rays));
+    NERF_HIP_TRY(R->need(R->counts, n_rays));
+    NERF_HIP_TRY(R->need(R->offsets, n_rays));
+    NERF_HIP_TRY(R->need(R->scan_tmp, scan_tmp_words(n_rays)));
+    NERF_HIP_TRY(R->need(R->total, 1));
     NERF_HIP_TRY(hipMemcpyAsync(R->cams.ptr, d->cameras, sizeof(NerfExtCamera) * d->view_count, hipMemcpyHostToDevice, st));
 
     OccView occ;
@@ -934,7 +946,7 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
     std::vector<Chunk> chunks;
     uint64_t total = 0, biggest = 0;
     const uint32_t n_blocks = (n_rays + kScanBlockRays - 1u) / kScanBlockRays;
-    NERF_HIP_TRY(R->scan_tmp.reserve(std::max<uint64_t>(scan_tmp_words(n_rays), n_blocks)));
+    NERF_HIP_TRY(R->need(R->scan_tmp, std::max<uint64_t>(scan_tmp_words(n_rays), n_blocks)));
     // With the default chunk size and at most kSlotMaxSteps steps per ray the
     // chunks are whole blocks of rays holding at most kSlotSamples slot
     // entries, each marched once into per-ray slots of 2^slot_shift
@@ -979,10 +991,10 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
             chunks.push_back(c);
         }
     }
-    NERF_HIP_TRY(R->samples.reserve(biggest));
-    NERF_HIP_TRY(R->field.reserve(biggest));
-    NERF_HIP_TRY(R->qlist.reserve(biggest));
-    if (!slots) NERF_HIP_TRY(R->qray.reserve(biggest));
+    NERF_HIP_TRY(R->need(R->samples, biggest));
+    NERF_HIP_TRY(R->need(R->field, biggest));
+    NERF_HIP_TRY(R->need(R->qlist, biggest));
+    if (!slots) NERF_HIP_TRY(R->need(R->qray, biggest));
 
     // Every field launch of the rounds reads its entries' rays from the round
     // list (qray), so the march writes no per-sample ray index.
@@ -996,12 +1008,8 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
     }
     const FieldWeights w{(const half_t*)d->model->density_params, (const half_t*)d->model->color_params};
     if (ref_model) {
-        NERF_HIP_TRY(R->ref_frags.reserve(64ull * kRefFragments));
+        NERF_HIP_TRY(R->need(R->ref_frags, 64ull * kRefFragments));
         NERF_HIP_TRY(ref_pack_weights(w.density, w.color, R->ref_frags.ptr, st));
-    }
-    if (!ref_model) {
-        in.narrow_end = narrow_levels(g, d->cameras, d->view_count, occ.omin, occ.omax);
-        if (slots) NERF_HIP_TRY(plan_cells(R, g, d->model->table, (uint64_t)n_rays << slot_shift, in, st));
     }
     const float3 bg = make_float3(d->background[0], d->background[1], d->background[2]);
     // Rounds: the schedule's round ends 256, 512, 1024, ... until every
@@ -1018,17 +1026,21 @@ NERF_API NerfStatus nerf_ext_render(NerfExtRenderer* R, const NerfExtRenderDesc*
     if (n_rounds >= 2u)
         for (int k = 0; k < 2; ++k, ++n_rounds) Es[n_rounds] = Es[n_rounds - 1u];
     const uint32_t chunk_rays_max = n_rays;
-    NERF_HIP_TRY(R->state.reserve(n_rays));
-    NERF_HIP_TRY(R->prog.reserve(n_rays));
-    NERF_HIP_TRY(R->list[0].reserve(chunk_rays_max));
-    NERF_HIP_TRY(R->list[1].reserve(chunk_rays_max));
-    NERF_HIP_TRY(R->n_active.reserve(2));
-    NERF_HIP_TRY(R->cnt.reserve(chunk_rays_max));
-    NERF_HIP_TRY(R->off.reserve(chunk_rays_max));
-    NERF_HIP_TRY(R->round_total.reserve(kMaxRounds));
-    NERF_HIP_TRY(R->keep.reserve(chunk_rays_max));
-    NERF_HIP_TRY(R->koff.reserve(chunk_rays_max));
-    NERF_HIP_TRY(R->keep_total.reserve(1));
+    NERF_HIP_TRY(R->need(R->state, n_rays));
+    NERF_HIP_TRY(R->need(R->prog, n_rays));
+    NERF_HIP_TRY(R->need(R->list[0], chunk_rays_max));
+    NERF_HIP_TRY(R->need(R->list[1], chunk_rays_max));
+    NERF_HIP_TRY(R->need(R->n_active, 2));
+    NERF_HIP_TRY(R->need(R->cnt, chunk_rays_max));
+    NERF_HIP_TRY(R->need(R->off, chunk_rays_max));
+    NERF_HIP_TRY(R->need(R->round_total, kMaxRounds));
+    NERF_HIP_TRY(R->need(R->keep, chunk_rays_max));
+    NERF_HIP_TRY(R->need(R->koff, chunk_rays_max));
+    NERF_HIP_TRY(R->need(R->keep_total, 1));
+    if (!ref_model) {  // after every buffer that the render needs
+        in.narrow_end = narrow_levels(g, d->cameras, d->view_count, occ.omin, occ.omax);
+        if (slots) NERF_HIP_TRY(plan_cells(R, g, d->model->table, (uint64_t)n_rays << slot_shift, in, st));
+    }
     in.sample_index     = R->qlist.ptr;
     in.sample_index_ray = slots ? nullptr : R->qray.ptr;  // slots: the ray from the index
     in.slot_rays        = slots;
@@ -1164,15 +1176,15 @@ NERF_API NerfStatus nerf_ext_render_uniform(NerfExtRenderer* R, const NerfExtMod
     const uint64_t blocks_per_chunk = std::max<uint64_t>(1u, kChunkSamples / ((uint64_t)samples_per_ray * kScanBlockRays));
     const uint32_t chunk_rays       = (uint32_t)std::min<uint64_t>(blocks_per_chunk * kScanBlockRays, (uint64_t)(n_rays + kScanBlockRays - 1u) / kScanBlockRays * kScanBlockRays);
     const uint64_t chunk_samples    = (uint64_t)chunk_rays * samples_per_ray;
-    NERF_HIP_TRY(R->cams.reserve(view_count));
-    NERF_HIP_TRY(R->rays.reserve(2ull * n_rays));
-    NERF_HIP_TRY(R->counts.reserve(n_rays));
-    NERF_HIP_TRY(R->offsets.reserve(n_rays));
-    NERF_HIP_TRY(R->scan_tmp.reserve(scan_tmp_words(chunk_rays)));
-    NERF_HIP_TRY(R->total.reserve(1));
-    NERF_HIP_TRY(R->samples.reserve(chunk_samples));
-    NERF_HIP_TRY(R->sample_ray.reserve(chunk_samples));
-    NERF_HIP_TRY(R->field.reserve(chunk_samples));
+    NERF_HIP_TRY(R->need(R->cams, view_count));
+    NERF_HIP_TRY(R->need(R->rays, 2ull * n_rays));
+    NERF_HIP_TRY(R->need(R->counts, n_rays));
+    NERF_HIP_TRY(R->need(R->offsets, n_rays));
+    NERF_HIP_TRY(R->need(R->scan_tmp, scan_tmp_words(chunk_rays)));
+    NERF_HIP_TRY(R->need(R->total, 1));
+    NERF_HIP_TRY(R->need(R->samples, chunk_samples));
+    NERF_HIP_TRY(R->need(R->sample_ray, chunk_samples));
+    NERF_HIP_TRY(R->need(R->field, chunk_samples));
     NERF_HIP_TRY(hipMemcpyAsync(R->cams.ptr, cameras, sizeof(NerfExtCamera) * view_count, hipMemcpyHostToDevice, st));
     const float3 bmin = make_float3(aabb6[0], aabb6[1], aabb6[2]), bmax = make_float3(aabb6[3], aabb6[4], aabb6[5]);
     k_uniform_rays<<<(n_rays + 255u) / 256u, 256, 0, st>>>(R->cams.ptr, W * H, n_rays, bmin, bmax, samples_per_ray, R->rays.ptr, R->counts.ptr);
@@ -1188,7 +1200,7 @@ NERF_API NerfStatus nerf_ext_render_uniform(NerfExtRenderer* R, const NerfExtMod
     }
     const FieldWeights w{(const half_t*)model->density_params, (const half_t*)model->color_params};
     if (ref_model) {
-        NERF_HIP_TRY(R->ref_frags.reserve(64ull * kRefFragments));
+        NERF_HIP_TRY(R->need(R->ref_frags, 64ull * kRefFragments));
         NERF_HIP_TRY(ref_pack_weights(w.density, w.color, R->ref_frags.ptr, st));
     }
     if (!ref_model) {
