@@ -58,6 +58,12 @@ NERF_API const char* nerf_ext_last_error(void);
 NERF_API NerfStatus nerf_ext_device_info(NerfExtDeviceInfo* out);
 NERF_API NerfStatus nerf_ext_malloc(void** out_ptr, uint64_t bytes);
 NERF_API NerfStatus nerf_ext_free(void* ptr);
+/* Point calls (nerf_ext_field_forward, the reference network's) take their
+ * temporary memory from a pool of the library's that keeps up to 192 MiB per GPU
+ * for the next call; this waits for the current GPU and gives it back.  The
+ * destroy calls of trainers and renderers do as well, and so does an allocation
+ * of the library that finds no memory. */
+NERF_API NerfStatus nerf_ext_release_scratch(void);
 NERF_API NerfStatus nerf_ext_memcpy(void* dst, const void* src, uint64_t bytes, uint32_t kind);
 NERF_API NerfStatus nerf_ext_memset(void* dst, int value, uint64_t bytes);
 NERF_API NerfStatus nerf_ext_synchronize(void);
@@ -349,7 +355,11 @@ typedef struct NerfExtRenderStats {
 NERF_API NerfStatus nerf_ext_renderer_create(NerfExtRenderer** out);
 NERF_API NerfStatus nerf_ext_renderer_destroy(NerfExtRenderer* renderer);
 /* Renders view_count views into rgba8 [view][H][W] (device), max_steps at
- * most 2^19.  Optional device
+ * most 2^19.  The renderer keeps its buffers until it is destroyed; a render of
+ * an fp16 table that may march 2^24 samples or more adds tables of up to
+ * 2.25 GiB, which it does without where memory is short.  Renders sum a cell's
+ * corners with one rounding per corner, points and training steps with two
+ * (images differ by about 1e-7 from the other sums).  Optional device
  * outputs: rgb_f32 [view][H][W][3] (unclamped composite) and counts
  * [view][H][W] (occupied samples per ray).  With stats != NULL the call
  * synchronises and times each stage with HIP events on desc->stream. */

@@ -324,6 +324,7 @@ PROTOTYPES: dict[str, tuple] = {
     "nerf_ext_device_info": (_S, [C.POINTER(NerfExtDeviceInfo)]),
     "nerf_ext_malloc": (_S, [C.POINTER(_P), _U64]),
     "nerf_ext_free": (_S, [_P]),
+    "nerf_ext_release_scratch": (_S, []),
     "nerf_ext_memcpy": (_S, [_P, _P, _U64, _U32]),
     "nerf_ext_memset": (_S, [_P, C.c_int, _U64]),
     "nerf_ext_synchronize": (_S, []),

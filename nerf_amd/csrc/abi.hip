@@ -118,12 +118,12 @@ NerfStatus Context::init_model() {
     const uint32_t nd = density_params(), nc = color_params();
     table_elems       = ref ? 0u : (uint64_t)grid_params.n_levels * grid_params.table_size * grid_params.n_features;
     if (!ref) {
-        NERF_HIP_TRY(hipMalloc(&table, table_elems * sizeof(uint16_t)));
-        NERF_HIP_TRY(hipMalloc(&table_f32, table_elems * sizeof(float)));
+        NERF_HIP_TRY(device_malloc((void**)&table, table_elems * sizeof(uint16_t)));
+        NERF_HIP_TRY(device_malloc((void**)&table_f32, table_elems * sizeof(float)));
     }
-    NERF_HIP_TRY(hipMalloc(&dparams, nd * sizeof(uint16_t)));
-    NERF_HIP_TRY(hipMalloc(&cparams, nc * sizeof(uint16_t)));
-    NERF_HIP_TRY(hipMalloc(&mlp_f32, (uint64_t)(nd + nc) * sizeof(float)));
+    NERF_HIP_TRY(device_malloc((void**)&dparams, nd * sizeof(uint16_t)));
+    NERF_HIP_TRY(device_malloc((void**)&cparams, nc * sizeof(uint16_t)));
+    NERF_HIP_TRY(device_malloc((void**)&mlp_f32, (uint64_t)(nd + nc) * sizeof(float)));
     if (!ref) {
         NerfExtGridDesc g32 = grid;
         g32.table_dtype     = NERF_EXT_F32;
@@ -222,18 +222,18 @@ NERF_API NerfStatus nerf_create_context(const NerfCreateDesc* desc, void** out_c
     const uint64_t cells = (uint64_t)d.occupancy_grid_res * d.occupancy_grid_res * d.occupancy_grid_res;
     NerfStatus s         = NERF_STATUS_OK;
     if (cells) {
-        if (hipMalloc(&ctx->bitfield, (cells + 31u) / 32u * 4u) != hipSuccess || hipMalloc(&ctx->density_grid, cells * sizeof(float)) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
+        if (device_malloc((void**)&ctx->bitfield, (cells + 31u) / 32u * 4u) != hipSuccess || device_malloc((void**)&ctx->density_grid, cells * sizeof(float)) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
         if (hipMemset(ctx->bitfield, 0, (cells + 31u) / 32u * 4u) != hipSuccess || hipMemset(ctx->density_grid, 0, cells * sizeof(float)) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
     }
     s = ctx->init_model();
     if (s != NERF_STATUS_OK) return NERF_STATUS_FAILURE;
     if (image_bytes) {
-        if (hipMalloc(&ctx->images, image_bytes) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
+        if (device_malloc((void**)&ctx->images, image_bytes) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
         if (hipMemcpy(ctx->images, d.images_rgba8, image_bytes, hipMemcpyHostToDevice) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
     }
     const uint64_t frame_bytes = (uint64_t)d.image_width * d.image_height * 4u;
     if (frame_bytes) {
-        if (hipMalloc(&ctx->rgba, frame_bytes) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
+        if (device_malloc((void**)&ctx->rgba, frame_bytes) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
         if (hipMemset(ctx->rgba, 0, frame_bytes) != hipSuccess) return NERF_STATUS_CUDA_ERROR;
     }
     if (nerf_ext_renderer_create(&ctx->renderer) != NERF_STATUS_OK) return NERF_STATUS_FAILURE;

@@ -648,13 +648,15 @@ uint32_t device_cu_count();
 // next call up to kScratchKept bytes per GPU, where the default pool gives it
 // back to the system at the next synchronisation and the call after that
 // allocates anew.  scratch_trim gives the current GPU's unused blocks back;
-// the destroy calls of the library's objects do, and an allocation that fails
-// does before it is tried once more.  Where the pool cannot be made the default
+// nerf_ext_release_scratch and the destroy calls of the library's objects do,
+// and an allocation of the library that fails does before it is tried once more
+// (device_malloc: hipMalloc with that).  Where the pool cannot be made the default
 // one serves.  Refused on a stream under capture: a graph that held the
 // allocation, replayed between eager calls, faulted the GPU.  Safe from any
 // thread, for any stream.
 constexpr uint64_t kScratchKept = 192ull << 20;
 hipError_t scratch_alloc(void** p, uint64_t bytes, hipStream_t stream);
 void scratch_trim();
+hipError_t device_malloc(void** p, uint64_t bytes);
 
 }  // namespace nerf_hip

@@ -635,7 +635,7 @@ struct NerfExtRenderer {
             ptr = nullptr;
             cap = 0;
             const uint64_t want = n + n / 8u + 256u;
-            hipError_t e        = hipMalloc(&ptr, want * sizeof(T));
+            hipError_t e        = nerf_hip::device_malloc((void**)&ptr, want * sizeof(T));
             if (e == hipSuccess) cap = want;
             return e;
         }

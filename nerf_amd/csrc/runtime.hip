@@ -95,6 +95,15 @@ hipError_t scratch_alloc(void** p, uint64_t bytes, hipStream_t stream) {
     return e;
 }
 
+hipError_t device_malloc(void** p, uint64_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    (void)hipDeviceSynchronize();  // released blocks may still be in use
+    scratch_trim();
+    return hipMalloc(p, bytes);
+}
+
 void scratch_trim() {
     hipMemPool_t pool = nullptr;
     if (scratch_pool(false, &pool) == hipSuccess && pool) (void)hipMemPoolTrimTo(pool, 0);
@@ -131,7 +140,13 @@ NERF_API NerfStatus nerf_ext_malloc(void** out_ptr, uint64_t bytes) {
     NERF_CHECK_ARG(out_ptr, "nerf_ext_malloc: null output");
     *out_ptr = nullptr;
     if (bytes == 0) return NERF_STATUS_OK;
-    NERF_HIP_TRY(hipMalloc(out_ptr, bytes));
+    NERF_HIP_TRY(device_malloc(out_ptr, bytes));
+    return NERF_STATUS_OK;
+}
+
+NERF_API NerfStatus nerf_ext_release_scratch(void) {
+    NERF_HIP_TRY(hipDeviceSynchronize());
+    scratch_trim();
     return NERF_STATUS_OK;
 }
 

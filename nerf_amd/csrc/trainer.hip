@@ -30,7 +30,7 @@ Trainer::~Trainer() {
 template <typename T>
 static hipError_t alloc(Trainer& t, T*& ptr, uint64_t count) {
     void* p        = nullptr;
-    const hipError_t e = hipMalloc(&p, count * sizeof(T) > 0 ? count * sizeof(T) : 16u);
+    const hipError_t e = device_malloc(&p, count * sizeof(T) > 0 ? count * sizeof(T) : 16u);
     if (e != hipSuccess) return e;
     t.owned.push_back(p);
     ptr = static_cast<T*>(p);

@@ -51,7 +51,7 @@ int hipMallocFromPoolAsync(void** p, size_t n, void* pool, void* stream) {
 }
 """
 
-CASES = ("tables_last", "tables_given_up", "field_without_memory")
+CASES = ("tables_last", "tables_given_up", "pool_given_back", "field_without_memory")
 
 
 def _render_setup():
@@ -108,6 +108,29 @@ def _run(case, shim):
         shim.shim_limit(before + total - tables + (1 << 20))
         assert np.array_equal(render(r, 3), want) and shim.shim_failed() > 0
         shim.shim_limit(-1)
+    elif case == "pool_given_back":
+        n = 4096
+        m = ext.RefModel.create(ext.ref_mlp_init(0), ext.ref_mlp_init(1))
+        p, d, o = DeviceArray.from_numpy(points(n, seed=1)), DeviceArray.from_numpy(unit_dirs(n, seed=2)), DeviceArray((n, 4), np.float32)
+        for _ in range(2):
+            L.call("nerf_ext_ref_field_forward", m.density.ptr, m.color.ptr, p.ptr, d.ptr, n, o.ptr, None, None)
+            synchronize()
+            L.call("nerf_ext_release_scratch")
+        out = C.c_void_p()
+        shim.shim_fail(1, 0)  # an allocation that fails once is tried again
+        L.call("nerf_ext_malloc", C.byref(out), 1 << 20)
+        assert out.value and shim.shim_failed() == 1
+        L.call("nerf_ext_free", out)
+        shim.shim_fail(2, 0)
+        with pytest.raises(L.NerfError):
+            L.call("nerf_ext_malloc", C.byref(out), 1 << 20)
+        shim.shim_fail(0, 1)
+        with pytest.raises(L.NerfError):
+            L.call("nerf_ext_ref_field_forward", m.density.ptr, m.color.ptr, p.ptr, d.ptr, n, o.ptr, None, None)
+        shim.shim_fail(0, 0)
+        L.call("nerf_ext_ref_field_forward", m.density.ptr, m.color.ptr, p.ptr, d.ptr, n, o.ptr, None, None)
+        synchronize()
+        assert np.any(o.numpy())
     else:
         n = 70001
         model = ext.Model.create(ext.grid_desc(18, L.NERF_EXT_F16), seed=1, table_range=1.0)
