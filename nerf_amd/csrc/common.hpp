@@ -265,7 +265,7 @@ bool make_occ_view(const NerfExtOccupancy& o, OccView& v);
 //     of that aligned entry pair; otherwise two single-entry loads (also
 //     merging the odd-x cases whose entries happen to be adjacent measured
 //     no faster).
-// Same entries, weights and summation order as encode_level.
+// Same entries, weights and summation order as the other gathers of a level.
 template <typename TableT, bool kHashPairs = true, bool kFma = false>
 __device__ __forceinline__ void encode_level_xpair(const GridParams& g, const TableT* __restrict__ table, const float p[3], uint32_t level, uint32_t N, bool dense, float& a0, float& a1) {
     const LevelCell c  = level_cell(p, N);
@@ -323,7 +323,7 @@ __device__ __forceinline__ void encode_level_xpair(const GridParams& g, const Ta
 // the odd lane's point, so each load instruction asks for one line per
 // point where one lane per point asks for two; a quad_perm swap per edge
 // then hands each lane the other half of its own point's corners.  Same
-// entries, weights and summation order as encode_level.
+// entries, weights and summation order as the other gathers of a level.
 __device__ __forceinline__ uint32_t pair_swap(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, false); }  // quad_perm [1, 0, 3, 2]
 
 // kWide: every load is 8 bytes (an fp32 entry, or the aligned pair that holds
@@ -614,15 +614,17 @@ hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_
 hipError_t launch_ref_density(const half8_t* frags, const FieldInputs& in, uint32_t n, half_t* dens_out, hipStream_t stream);
 // Workgroups, and partials, of the weight-gradient kernels.
 uint32_t ref_grad_blocks(uint32_t np);
-// Training of the reference model (the trainer's stages).  Rows of the
-// neuron-major fp16 buffers (blocks of 32 samples) the backward writes per sample: every layer's
-// input (acts) and output delta (dlts); weight-gradient partials per chunk of
-// kRefDwChunk samples; kRefReduceBlocks squared-norm partials.
+// Rows of the neuron-major fp16 buffers (blocks of 32 samples) that
+// nerf_ext_ref_backward_rows writes per sample: every layer's input (acts) and
+// output delta (dlts); samples per partial of its weight gradients.
 constexpr uint32_t kRefActRows = 1136u, kRefDltRows = 1056u;
 constexpr uint32_t kRefDwChunk = 4096u;
 constexpr uint32_t kRefParams = NERF_EXT_REF_DENSITY_PARAMS + NERF_EXT_REF_COLOR_PARAMS;
-constexpr uint32_t kRefReduceBlocks = (kRefParams + 255u) / 256u;  // one parameter per thread
-constexpr uint32_t kRefMaxSamples = 1u << 20;  // per backward call: the buffers stay below 4 GiB (buffer-descriptor range)
+constexpr uint32_t kRefReduceBlocks = (kRefParams + 255u) / 256u;  // one parameter per thread, one squared-norm partial per block
+// Samples per backward call, with and without rows, and per training step: the
+// row buffers stay below the 4 GiB that a buffer descriptor addresses.
+constexpr uint32_t kRefMaxSamples = 1u << 20;
+// Training of the reference model (the trainer's stages).
 struct RefTrainLaunch {
     half8_t* frags;    // 64 x kRefFragments
     half_t* dens;      // [np][16] density outputs: the forward's, or of launch_ref_density where no forward went before

@@ -1487,7 +1487,7 @@ hipError_t launch_ref_field(const half8_t* frags, const FieldInputs& in, uint32_
     return hipGetLastError();
 }
 
-static_assert(kActRows == kRefActRows && kDltRows == kRefDltRows, "training buffer rows");
+static_assert(kActRows == kRefActRows && kDltRows == kRefDltRows, "row buffers");
 
 hipError_t launch_ref_density(const half8_t* frags, const FieldInputs& in, uint32_t n, half_t* dens_out, hipStream_t stream) {
     if (n == 0u) return hipSuccess;
@@ -1570,7 +1570,7 @@ NerfStatus ref_backward(const char* who, const uint16_t* density_params, const u
                         float* dcolor, uint16_t* acts_out, uint16_t* dlts_out, void* stream) {
     if (n == 0u) return NERF_STATUS_OK;
     NERF_CHECK_ARG(density_params && color_params && positions && directions && draw && ddensity && dcolor, std::string(who) + ": null pointer");
-    NERF_CHECK_ARG(n <= (1u << 20), std::string(who) + ": at most 2^20 samples per call (buffer descriptors address < 4 GiB)");
+    NERF_CHECK_ARG(n <= kRefMaxSamples, std::string(who) + ": at most 2^20 samples per call");
     hipStream_t st        = (hipStream_t)stream;
     const uint32_t np     = (n + 63u) / 64u * 64u;
     const bool rows       = acts_out != nullptr;  // with rows: stored, and multiplied from there

@@ -95,11 +95,11 @@ def test_field_forward(log2_t, dtype):
 
 @pytest.mark.parametrize("log2_t,dtype", [(19, L.NERF_EXT_F16), (17, L.NERF_EXT_F32)])
 def test_field_forward_level_major_launch(log2_t, dtype):
-    # More than 2^20 points take the level-major field kernel (renders); the
-    # smaller launches above take the tile kernel.  Rows compared with the
-    # oracle on a sample; the first 2^20 rows bit for bit with the tile
-    # kernel (the same fp32 feature sums in the oracle's order, the same MFMA
-    # chain), whatever lanes fetch which corners.
+    # More than 2^20 points take the level-major field kernel; launches of at
+    # most 2^16 take the tile kernel.  Rows compared with the oracle on a
+    # sample; the first 2^20 rows bit for bit with the tile kernel (the same
+    # fp32 feature sums in the oracle's order, the same MFMA chain), whatever
+    # lanes fetch which corners.
     n = (1 << 20) + 4099
     announce(f"field forward level-major n={n} log2_t={log2_t} dtype={dtype}")
     desc = ext.grid_desc(log2_t, dtype)
@@ -110,7 +110,8 @@ def test_field_forward_level_major_launch(log2_t, dtype):
     ms = model.struct()
     L.call("nerf_ext_field_forward", byref(ms), d_pos.ptr, d_dir.ptr, n, d_o.ptr, None)
     d_tile = DeviceArray((1 << 20, 4), np.float32)
-    L.call("nerf_ext_field_forward", byref(ms), d_pos.ptr, d_dir.ptr, 1 << 20, d_tile.ptr, None)
+    for a in range(0, 1 << 20, 1 << 16):
+        L.call("nerf_ext_field_forward", byref(ms), d_pos.ptr + 12 * a, d_dir.ptr + 12 * a, 1 << 16, d_tile.ptr + 16 * a, None)
     synchronize()
     got = d_o.numpy()
     rows = np.unique(np.concatenate([np.random.default_rng(5).integers(0, n, 4000), np.arange(n - 70, n)]))

@@ -1,5 +1,7 @@
 """GPU scene, occupancy, march and render parity.  Occupancy bits and per-ray
 sample counts bit-exact; RGB within 1e-3 relative; RGBA8 within 1 LSB."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -172,3 +174,24 @@ def test_render_is_the_same_from_every_field_kernel(dtype, log2_t, width, height
         outs.append((rgba.numpy(), rgb.numpy().view(np.uint32)))
     for other in outs[1:]:
         assert np.array_equal(outs[0][0], other[0]) and np.array_equal(outs[0][1], other[1])
+
+
+@pytest.mark.parametrize("log2_t", [15, 19])
+def test_render_uniform_with_cell_tables(log2_t):
+    # 2^24 possible samples or more: uniform sampling gathers its leading levels
+    # from cell tables and its other coherent ones by narrow loads.
+    w, h, spp, bg = 421, 319, 125, (0.2, 0.5, 0.9)
+    assert w * h * spp >= 1 << 24
+    announce(f"nerf_ext_render_uniform {w}x{h} at {spp} samples, T=2^{log2_t}, against the oracle on a subset of rays")
+    desc = ext.grid_desc(log2_t, L.NERF_EXT_F16)
+    model = ext.Model.create(desc, seed=7, table_range=1.0)
+    dp, cp = host_params(model)
+    cams = (L.NerfExtCamera * 1)(ext.camera_orbit(0, 2, 1.32, CENTRE, w, h, 1111.0 * w / 800.0))
+    r, ms, rgba, rgb = ext.Renderer(), model.struct(), DeviceArray((h, w), np.uint32), DeviceArray((h, w, 3), np.float32)
+    L.call("nerf_ext_render_uniform", r._h, byref(ms), cams, 1, C.cast((C.c_float * 6)(*BOX), C.c_void_p), spp, C.cast((C.c_float * 3)(*bg), C.c_void_p), rgba.ptr, rgb.ptr, None)
+    synchronize()
+    rays = np.append(np.arange(0, w * h, 499, dtype=np.uint32), np.uint32(w * h - 1))
+    want_rgb, want_rgba, counts = orc.render_uniform(oracle_grid(desc), host_table(model), dp, cp, orc.camera_from_bytes(bytes(cams[0])), BOX, spp, rays, bg=bg, threads=8, kind=0)
+    assert (counts == spp).mean() > 0.3
+    assert_rel(rgb.numpy().reshape(-1, 3)[rays], want_rgb, what="uniform render rgb")
+    assert np.abs(rgba.numpy().ravel()[rays].view(np.uint8).astype(int) - want_rgba.view(np.uint8).astype(int)).max() <= 1
